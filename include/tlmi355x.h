@@ -107,15 +107,16 @@ int tlm_rope(const void* q, const void* k, const void* cos_t, const void* sin_t,
  * in_dtype: F16 | BF16; out_dtype: F16 | BF16 | F32. The fp32 program
  * (tpu_demo/matmul/tpu_test_matmul_fp32.py:9-31) copies its fp32 A/B tiles to fp16 before
  * ppl_gemm: tlm_cast to F16, then this with out_dtype F32.
- * M <= 16 with trans_b == 0 (and with trans_b == 1 when the output has few 64-column strips)
- * splits K over several workgroups whose partial tiles meet in a library-owned device workspace (16 MB per GPU, 4 slots): each stream owns one slot, so calls
- * on one stream are ordered and calls that overlap use different slots; further streams take an
- * unsplit kernel. A HIP graph keeps the slot of the stream it was captured on, so its replays
- * must not overlap each other or other work of that stream. Slots are keyed by the stream handle:
- * a stream created after another is destroyed can get the same handle and inherits its slot, so
- * a stream is destroyed only once its calls have finished. The result does not depend on the
- * split's timing: a stream's calls are bitwise reproducible (the unsplit kernel of a stream
- * without a slot sums in another order, so its last bits can differ from the split kernel's). */
+ * Calls whose tiles are fewer than the CUs split K over several workgroups, whose partial tiles
+ * meet in a library-owned device workspace (64 MB per GPU, 4 slots): each stream owns one slot,
+ * so calls on one stream are ordered and calls that overlap use different slots; further streams
+ * (and hipStreamPerThread) run unsplit. Inside a stream capture only M <= 16 may split: such a HIP
+ * graph keeps the slot of the stream it was captured on, so its replays must not overlap each
+ * other or other work of that stream; larger calls are captured unsplit. Slots are keyed by the
+ * stream handle: a stream created after another is destroyed can get the same handle and inherits
+ * its slot, so a stream is destroyed only once its calls have finished. The result does not depend
+ * on the split's timing: a stream's calls are bitwise reproducible (a call that runs unsplit sums
+ * in another order, so its last bits can differ from a split one's). */
 int tlm_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int in_dtype,
              int out_dtype, int trans_b, void* stream);
 
@@ -124,7 +125,8 @@ int tlm_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_
  * Reference: examples/gemm_fp8/example_tilelang_gemm_fp8.py:17-37 (T.gemm transpose_B=True,
  * fp8 C; oracle (a.half() @ b.half().T).to(fp8), :46-55) and example_tilelang_gemm_fp8_2xAcc.py
  * (fp32 C). in_dtype: F8E4M3 | F8E5M2 (OCP); out_dtype: F32 | F16 | BF16 | in_dtype (round to
- * nearest even without saturation, as torch's cast). */
+ * nearest even without saturation, as torch's cast). Shapes with few tiles split K through the
+ * workspace of tlm_gemm under the same rules, but never inside a stream capture. */
 int tlm_gemm_fp8(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
                  int in_dtype, int out_dtype, int trans_b, void* stream);
 

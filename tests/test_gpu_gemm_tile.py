@@ -1,0 +1,114 @@
+"""GPU parity of the tiles between one decode step and a whole prompt batch (tlm_gemm_tile.h): sizes
+at the edges of every tile (32, 64, 128, 256 rows; 64 and 128 columns; 64- and 128-value k-tiles),
+remainders on each axis, and K splits, against the fp64 product of the same inputs.
+
+Tolerance: fp32 sums of K products with |partial sums| <= s err by at most K ulp(s) / 2; here the
+relative 2-norm error stays below 4 sqrt(K) 2^-24, plus half an ulp of the output type (2^-9 bf16,
+2^-12 fp16). fp8 above 16 rows: the fp8 matrix instruction drops low bits of its sums (measured 1.3e-5).
+"""
+import pytest
+import torch
+
+from tilelang.jit.adapter.mi355x import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+ULP = {torch.float32: 0.0, torch.float16: 2.0 ** -12, torch.bfloat16: 2.0 ** -9}
+
+
+def _rel(c, exp):
+    return float((c.double() - exp).norm() / exp.norm())
+
+
+def _run(M, N, K, dt, out, trans_b, seed=0, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed + M + N + K)
+    a = torch.randn(M, K, generator=g, device=DEV).to(dt)
+    b = torch.randn(*((N, K) if trans_b else (K, N)), generator=g, device=DEV).to(dt)
+    c = torch.full((M, N), float("nan"), device=DEV).to(out)
+    ops.gemm(a, b, c, trans_b=trans_b)
+    bd = b.double()
+    return c, a.double() @ (bd.T if trans_b else bd)
+
+
+SHAPES = [(17, 64, 64), (32, 136, 200), (33, 64, 4096), (64, 2048, 1000), (65, 520, 2048),
+          (128, 128, 7168), (129, 1032, 776), (200, 4096, 264), (257, 640, 4096), (500, 4096, 1024),
+          (1000, 1024, 520), (1025, 4096, 128), (1, 2048, 2048), (16, 520, 72), (5, 28672, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("dt,out,trans_b", [(torch.bfloat16, torch.bfloat16, False),
+                                            (torch.float16, torch.float32, True),
+                                            (torch.float16, torch.float16, True),
+                                            (torch.bfloat16, torch.float32, False)])
+def test_gemm_tiles(M, N, K, dt, out, trans_b):
+    c, exp = _run(M, N, K, dt, out, trans_b)
+    assert _rel(c, exp) < 4 * K ** 0.5 * 2.0 ** -24 + ULP[out]
+
+
+@pytest.mark.parametrize("M,N,K", [(20, 77, 64), (70, 1001, 520), (130, 131, 2056)])
+def test_gemm_tiles_bt_any_column_count(M, N, K):
+    """B^T takes any N: the last columns leave as single values."""
+    for out in (torch.float16, torch.float32):
+        c, exp = _run(M, N, K, torch.float16, out, True)
+        assert _rel(c, exp) < 4 * K ** 0.5 * 2.0 ** -24 + ULP[out]
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 512, 4096), (16, 1000, 528), (17, 64, 128), (64, 2048, 2000),
+                                   (65, 520, 1024), (300, 1040, 784), (512, 4096, 512)])
+@pytest.mark.parametrize("dt", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_gemm_fp8_tiles(M, N, K, dt):
+    """16 rows or fewer are multiplied as fp16: fp32 sums, no low bits dropped."""
+    c, exp = _run(M, N, K, dt, torch.float32, True)
+    assert _rel(c, exp) < 4 * K ** 0.5 * 2.0 ** -24 + (0 if M <= 16 else 5e-5)
+
+
+def test_gemm_fp8_few_rows_keep_specials():
+    """inf, NaN and subnormals of both formats through the fp16 product."""
+    for dt in (torch.float8_e4m3fn, torch.float8_e5m2):
+        a = torch.eye(16, 256, device=DEV).to(dt)
+        codes = torch.arange(256, dtype=torch.uint8, device=DEV).view(1, 256).repeat(64, 1)
+        b = torch.zeros(64, 256, dtype=dt, device=DEV)
+        for i in range(16):  # column k of B^T holds 64 consecutive codes, one k per row of A
+            b.view(torch.uint8)[:, i] = codes[0, (16 * torch.arange(64, device=DEV) + i) % 256]
+        c = torch.empty(16, 64, device=DEV)
+        ops.gemm(a, b, c, trans_b=True)
+        exp = b.float()[:, :16].T
+        finite = torch.isfinite(b.float()).all(1)  # 0 * inf = NaN in a row with a special
+        assert torch.equal(c[:, finite], exp[:, finite])
+        assert not torch.isfinite(c[:, ~finite]).any()
+
+
+def test_gemm_split_tiles_repeat_and_replay():
+    """A split call gives the same bits again, with other calls between; captured, it runs unsplit, so two graphs
+    of one capture stream may replay at the same time on two streams."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    a = [torch.randn(64, 4096, generator=g, device=DEV).half() for _ in range(2)]
+    b = torch.randn(1024, 4096, generator=g, device=DEV).half()
+    eager = []
+    for x in a:
+        for _ in range(2):
+            c = torch.empty(64, 1024, device=DEV)
+            ops.gemm(x, b, c, trans_b=True)
+            eager.append(c)
+            ops.gemm(x[:20], b[:200], torch.empty(20, 200, device=DEV), trans_b=True)
+    assert torch.equal(eager[0], eager[1]) and torch.equal(eager[2], eager[3])
+    side = torch.cuda.Stream()
+    outs, graphs = [torch.zeros(64, 1024, device=DEV) for _ in a], []
+    side.wait_stream(torch.cuda.current_stream())
+    for x, c in zip(a, outs):
+        gr = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(gr, stream=side):
+            ops.gemm(x, b, c, trans_b=True)
+        graphs.append(gr)
+    streams = [torch.cuda.Stream() for _ in a]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        for gr, st in zip(graphs, streams):
+            with torch.cuda.stream(st):
+                gr.replay()
+        torch.cuda.synchronize()
+        for c, e in zip(outs, (eager[0], eager[2])):
+            assert _rel(c, e.double()) < 4 * 64 * 2.0 ** -24
+        for c in outs:
+            c.zero_()
+        torch.cuda.synchronize()

@@ -20,9 +20,9 @@
 //   * workgroup -> tile order is XCD-aware: consecutive workgroup ids land on different XCDs
 //     (round-robin dispatch), so ids are regrouped to give each XCD a compact block of tiles
 //     that shares A row-panels and B column-panels in that XCD's L2.
-// Skinny kernels (M <= 16): gemm_skinny_split for row-major B, gemm_skinny for B^T and the shapes
-// or streams the split kernel does not take; see below.
-#include "tlm_common.h"
+// gemm_skinny_split: 16 rows or fewer on a large row-major B. Everything between (and B^T at any
+// row count that 256x256 tiles do not fill the chip with): the tiles of tlm_gemm_tile.h.
+#include "tlm_gemm_tile.h"
 
 #include <algorithm>
 #include <mutex>
@@ -408,166 +408,6 @@ __global__ __launch_bounds__(NTHREADS, 1) void gemm_256x256(const uint16_t* __re
 }
 
 // ------------------------------------------------------------------------------------------------
-// Skinny GEMM (M <= 16) for B^T and the row-major cases gemm_skinny_split does not take: the
-// whole of A fits one MFMA row block, so the kernel streams B.
-// Workgroup = 8 waves on a 64-column strip of C; the waves split K into interleaved 32-row
-// blocks, each block is one v_mfma_f32_16x16x32 per 16 columns. A operand (row m = lane%16,
-// k = 8*(lane/16)..+7) is a direct 16-byte global load. Row-major B goes through a wave-private
-// LDS buffer [32][64] and comes back through ds_read_b64_tr_b16; B^T ([N,K]) is loaded straight
-// into operand layout. The next block's loads are issued before the current block's MFMAs.
-// The 8 partial 16x64 tiles are summed through LDS at the end. B is read once per call, with
-// non-temporal loads: 3% faster back to back, and a single launch after a cache flush 27 against
-// 48 us at 16 x 14336 x 4096. With nsplit > 1 (B^T with few strips) the workgroups of a strip
-// take 1/nsplit of K each and their tiles meet as in gemm_skinny_split (split order, last
-// arriver).
-constexpr int SS_WAVES = 8;
-constexpr int SS_NT = 128;
-constexpr int SS_BK = 16;
-constexpr int SS_AMAX_K = 2048;  // k range of one workgroup: its A is 64 KB of LDS
-constexpr int SS_MAX_SPLIT = 16;
-constexpr int SS_SLOTS = 4;
-constexpr int SS_MAX_WG = 512;   // workgroups of one call that publish a partial tile
-constexpr int SS_PART = 16 * SS_NT;
-constexpr int SK_WAVES = 8;
-constexpr int SK_NT = 64;
-constexpr int SK_BK = 32;
-constexpr int SK_BPITCH = SK_NT + 16;  // halves per LDS row of a B block (160 bytes)
-
-
-template <bool BF16, bool TRANS_B, int OUT>
-__global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny(const uint16_t* __restrict__ A,
-                                                            const uint16_t* __restrict__ B,
-                                                            void* __restrict__ C, int M, int N,
-                                                            int K, int nsplit, float* part,
-                                                            unsigned* arrivals) {
-  using MT = mfma16_t<BF16>;
-  using v8 = typename MT::v8;
-  __shared__ __attribute__((aligned(16))) uint16_t sbuf[SK_WAVES][SK_BK * SK_BPITCH];
-  __shared__ float red[SK_WAVES][16][SK_NT + 1];
-  __shared__ unsigned last_arrival;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nstrips = (N + SK_NT - 1) / SK_NT;
-  const int strip = blockIdx.x % nstrips, split = blockIdx.x / nstrips;
-  const int n0 = strip * SK_NT;
-  const int KBall = (K + SK_BK - 1) / SK_BK;
-  const int kb_lo = (int)((int64_t)split * KBall / nsplit);
-  const int KB = (int)((int64_t)(split + 1) * KBall / nsplit);  // this split's blocks end
-  const int am = lane & 15, ak = 8 * (lane >> 4);
-  // row-major B block loads: 32 rows x 64 cols = 4 vectors per lane (rows lane/8 + 8p)
-  const int br = lane >> 3, bc = (lane & 7) * 8;
-  const int h = lane >> 4, j = lane & 15;
-
-  f32x4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = f32x4{};
-
-  u32x4 ra, rb[4];
-  auto load = [&](int kb) {
-    const int k0 = kb * SK_BK;
-    ra = (am < M && k0 + ak < K) ? *(const u32x4*)(A + (int64_t)am * K + k0 + ak)
-                                 : u32x4{0, 0, 0, 0};
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      if constexpr (TRANS_B) {
-        const int gn = n0 + 16 * p + am;
-        rb[p] = (gn < N && k0 + ak < K) ? ld_nt((const u32x4*)(B + (int64_t)gn * K + k0 + ak))
-                                        : u32x4{0, 0, 0, 0};
-      } else {
-        const int gk = k0 + br + 8 * p, gn = n0 + bc;
-        rb[p] = (gk < K && gn < N) ? ld_nt((const u32x4*)(B + (int64_t)gk * N + gn))
-                                   : u32x4{0, 0, 0, 0};
-      }
-    }
-  };
-
-  uint16_t* my = sbuf[wave];
-  int kb = kb_lo + wave;
-  if (kb < KB) load(kb);
-  for (; kb < KB; kb += SK_WAVES) {
-    const u32x4 ca = ra;
-    u32x4 cb[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) cb[p] = rb[p];
-    if (kb + SK_WAVES < KB) load(kb + SK_WAVES);
-    const v8 av = __builtin_bit_cast(v8, ca);
-    if constexpr (TRANS_B) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) acc[t] = MT::mma(av, __builtin_bit_cast(v8, cb[t]), acc[t]);
-    } else {
-#pragma unroll
-      for (int p = 0; p < 4; ++p) *(u32x4*)(my + (br + 8 * p) * SK_BPITCH + bc) = cb[p];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        // 16-lane group h reads k rows 8h + (j/4) (+4), columns 16t + 4*(j%4)
-        const uint16_t* p = my + (8 * h + (j >> 2)) * SK_BPITCH + 16 * t + 4 * (j & 3);
-        const v8 bv = cat4<v8>(lds_read_tr16(p), lds_read_tr16(p + 4 * SK_BPITCH));
-        acc[t] = MT::mma(av, bv, acc[t]);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-  }
-  // lane holds column 16t + lane%16, rows 4*(lane/16) + i
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) red[wave][4 * (lane >> 4) + i][16 * t + (lane & 15)] = acc[t][i];
-  __syncthreads();
-  constexpr int PER = 16 * SK_NT / (64 * SK_WAVES);  // outputs per thread
-  float v[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int o = threadIdx.x + i * 64 * SK_WAVES, r = o / SK_NT, c = o % SK_NT;
-    float s = 0.f;
-#pragma unroll
-    for (int w = 0; w < SK_WAVES; ++w) s += red[w][r][c];
-    v[i] = s;
-  }
-  if (nsplit > 1) {
-    // the strip's tiles meet in the workspace: sc0 sc1 stores (written through), a wait for
-    // them before the arrival, sc0 sc1 loads (missing every cache) after it; the sum runs in
-    // split order
-    const __amdgpu_buffer_rsrc_t rp =
-        __builtin_amdgcn_make_buffer_rsrc(part, (short)0, 0x7fffffff, RSRC_WORD3);
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-      __builtin_amdgcn_raw_buffer_store_b32(
-          __builtin_bit_cast(uint32_t, v[i]), rp,
-          (int)((blockIdx.x * SS_PART + threadIdx.x + i * 64 * SK_WAVES) * 4), 0, CP_SC01);
-    __builtin_amdgcn_s_waitcnt(0x3f70);  // vmcnt(0): the tile has been written
-    __syncthreads();
-    if (threadIdx.x == 0)
-      last_arrival = atomicAdd(&arrivals[strip], 1u) == (unsigned)(nsplit - 1);
-    __syncthreads();
-    if (!last_arrival) return;
-    float t[PER] = {};
-    for (int sp = 0; sp < nsplit; ++sp) {  // uniform
-#pragma unroll
-      for (int i = 0; i < PER; ++i) {
-        float x = v[i];
-        if (sp != split)
-          x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-              rp, (int)(((sp * nstrips + strip) * SS_PART + threadIdx.x + i * 64 * SK_WAVES) * 4),
-              0, CP_SC01));
-        t[i] += x;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < PER; ++i) v[i] = t[i];
-    if (threadIdx.x == 0) atomicExch(&arrivals[strip], 0u);
-  }
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int o = threadIdx.x + i * 64 * SK_WAVES, r = o / SK_NT, c = o % SK_NT;
-    if (r < M && n0 + c < N) store_out<OUT>(C, (int64_t)r * N + n0 + c, v[i]);
-  }
-}
-
-// ------------------------------------------------------------------------------------------------
 // Split skinny GEMM (M <= 16, row-major B): the preferred form of the M <= 16 stream. B is read
 // in 256-byte row segments (a 128-column strip per workgroup), and the k range is split over
 // `nsplit` workgroups per strip so that about one workgroup runs per CU. Measured on the bare
@@ -584,8 +424,17 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny(const uint16_t* __r
 // adds the tiles in split order (the result does not depend on arrival order), writes C and
 // resets the counter to zero. The workspace is a file-scope device array with SS_SLOTS slots;
 // each stream that runs this kernel on a device owns one slot, so calls that overlap are on
-// different streams and never share a slot. A further stream takes gemm_skinny. A HIP graph
+// different streams and never share a slot. A further stream takes an unsplit tile (tlm_gemm_tile.h). A HIP graph
 // keeps the slot of the stream it was captured on.
+
+constexpr int SS_WAVES = 8;
+constexpr int SS_NT = 128;
+constexpr int SS_BK = 16;
+constexpr int SS_AMAX_K = 2048;  // k range of one workgroup: its A is 64 KB of LDS
+constexpr int SS_MAX_SPLIT = 16;
+constexpr int SS_SLOTS = 4;      // workspace slots, one per stream
+constexpr int SS_MAX_WG = 512;   // workgroups of one call that publish a partial tile
+constexpr int SS_PART = 16 * SS_NT;
 
 template <bool BF16>
 struct mfma16k16_t;
@@ -780,12 +629,14 @@ __global__ __launch_bounds__(256) void gemm_generic(const uint16_t* __restrict__
 
 }  // namespace
 
-// Workspace of gemm_skinny_split, one instance per GPU (a device that loads this code object
-// holds its own copy until the process ends; 16 MB): SS_SLOTS slots of partial tiles and arrival
+// Workspace of the split kernels, one instance per GPU (a device that loads this code object
+// holds its own copy until the process ends; 64 MB): SS_SLOTS slots of partial tiles and arrival
 // counters. The counters start at zero and every call leaves them at zero. In host code the names
 // only identify the symbols; the device addresses come from hipGetSymbolAddress.
-static __device__ __align__(256) float ss_partials[SS_SLOTS][SS_MAX_WG][SS_PART];
-static __device__ __align__(256) unsigned ss_arrivals[SS_SLOTS][SS_MAX_WG];
+static __device__ __align__(256) float ss_partials[SS_SLOTS][TLM_SPLIT_BYTES / 4];
+static __device__ __align__(256) unsigned ss_arrivals[SS_SLOTS][TLM_SPLIT_TILES];
+static_assert(SS_MAX_WG <= TLM_SPLIT_TILES && (size_t)SS_MAX_WG * SS_PART * 4 <= TLM_SPLIT_BYTES,
+              "the skinny kernel's tiles fit a slot");
 
 namespace {
 
@@ -801,10 +652,11 @@ struct SsDevice {
 SsDevice g_ss[kSsDevices];
 std::mutex g_ss_mu;
 
+}  // namespace
+
 // The workspace slot of stream `s` on the current device: the one it owns, else a free one that
-// it then owns. False when every slot is owned by another stream (or the lookup failed), and the
-// caller takes gemm_skinny.
-bool ss_slot(hipStream_t s, float** part, unsigned** arrivals) {
+// it then owns. False when every slot is owned by another stream (or the lookup failed).
+bool tlm_split_slot(hipStream_t s, float** part, unsigned** arrivals) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kSsDevices) return false;
   SsDevice& d = g_ss[dev];
@@ -828,10 +680,12 @@ bool ss_slot(hipStream_t s, float** part, unsigned** arrivals) {
       slot = i;
     }
   if (slot < 0) return false;
-  *part = d.part + (size_t)slot * SS_MAX_WG * SS_PART;
-  *arrivals = d.arrivals + (size_t)slot * SS_MAX_WG;
+  *part = d.part + (size_t)slot * (TLM_SPLIT_BYTES / 4);
+  *arrivals = d.arrivals + (size_t)slot * TLM_SPLIT_TILES;
   return true;
 }
+
+namespace {
 
 // Split count of gemm_skinny_split for N x K (0: the shape does not fit it): about one
 // workgroup per CU without a second round, at least 16 blocks (256 k) and at most SS_AMAX_K of
@@ -846,36 +700,27 @@ int ss_nsplit(int N, int K) {
   return ns;
 }
 
-// Split count of gemm_skinny for B^T (1: no split): about one workgroup per CU when the 64-column
-// strips are fewer, at least 8 blocks (256 k) per workgroup.
-int sk_nsplit(int N, int K) {
-  const int nstrips = (N + SK_NT - 1) / SK_NT;
-  const int KB = (K + SK_BK - 1) / SK_BK;
-  int ns = std::max(1, std::min(SS_MAX_SPLIT, 256 / nstrips));
-  ns = std::min(ns, std::max(1, KB / 8));
-  return (int64_t)nstrips * ns > SS_MAX_WG ? 1 : ns;
-}
-
 template <bool BF16, bool TRANS_B, int OUT>
 int launch(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t s) {
   const bool vec = tlm_aligned(A, 16) && tlm_aligned(B, 16) && K % 8 == 0 &&
                    (TRANS_B || N % 8 == 0);
+  // One decode step on a large row-major B: the split skinny kernel streams 256-byte rows with A
+  // kept in LDS (16 rows: 4096 x 14336 23.5 us against 25.5 on the best tile, 14336 x 4096 24.4
+  // against 24.9). Below 32 MB the 32-row tile's shorter start and end win (4096^2 11.6 against
+  // 11.7, 2048^2 8.6 against 6.7, 512 x 4096 8.4 against 6.7).
   int ns = 0;
   float* part = nullptr;
   unsigned* arrivals = nullptr;
-  if (vec && M <= 16 && !TRANS_B && K > 0 && (int64_t)(K + 2 * SS_BK) * N * 2 < 0x7ffffff0)
+  if (vec && M <= 16 && !TRANS_B && (int64_t)N * K * 2 >= (32 << 20) &&
+      (int64_t)(K + 2 * SS_BK) * N * 2 < 0x7ffffff0)
     ns = ss_nsplit(N, K);
-  if (ns > 1 && !ss_slot(s, &part, &arrivals)) ns = 0;
+  if (ns > 1 && !tlm_split_slot(s, &part, &arrivals)) ns = 0;
   if (ns > 0) {
     const int nstrips = (N + SS_NT - 1) / SS_NT;
     gemm_skinny_split<BF16, OUT><<<(unsigned)(nstrips * ns), 64 * SS_WAVES, 0, s>>>(
         (const uint16_t*)A, (const uint16_t*)B, C, M, N, K, ns, part, arrivals);
-  } else if (vec && M <= 16) {
-    int nk = TRANS_B ? sk_nsplit(N, K) : 1;
-    if (nk > 1 && !ss_slot(s, &part, &arrivals)) nk = 1;
-    gemm_skinny<BF16, TRANS_B, OUT><<<(unsigned)((N + SK_NT - 1) / SK_NT * nk), 64 * SK_WAVES, 0,
-                                      s>>>((const uint16_t*)A, (const uint16_t*)B, C, M, N, K, nk,
-                                           part, arrivals);
+  } else if (vec && gt::run_tiles<BF16 ? gt::EL_BF16 : gt::EL_F16, TRANS_B, OUT>(A, B, C, M, N, K, s)) {
+    // between one decode step and a whole prompt batch
   } else if (vec && (int64_t)BM * K * 2 < 0x7ffffff0 &&
              (TRANS_B ? (int64_t)BN * K * 2 : (int64_t)BK * N * 2) < 0x7ffffff0) {
     // the LDS-DMA offsets of a 256-row panel (or a 64-row k-tile of row-major B) are 32-bit

@@ -12,7 +12,7 @@
 // one v_mfma_f32_16x16x128_f8f6f4 covers the whole k-tile for a 16x16 output tile at twice the
 // 16-bit FLOP rate. Each lane holds 32 bytes of its row (A) / column (B) l % 16: the 16-byte
 // chunks q and q + 4 of the row, q = l / 16.
-#include "tlm_common.h"
+#include "tlm_gemm_tile.h"
 
 #include <type_traits>
 
@@ -361,11 +361,13 @@ __global__ __launch_bounds__(256) void gemm8_generic(const uint8_t* __restrict__
 template <int FMT, int OUT>
 int launch(const void* A, const void* B, void* C, int M, int N, int K, bool trans_b,
            hipStream_t s) {
+  const bool vec = trans_b && K % 16 == 0 && tlm_aligned(A, 16) && tlm_aligned(B, 16);
   // 32-bit LDS-DMA byte offsets r * K + 16 c within a 256-row panel stay below the
   // descriptor's num_records (2^31 - 16): K < 2^23
-  const bool tiled = trans_b && M > 16 && K % 16 == 0 && K < (1 << 23) && tlm_aligned(A, 16) &&
-                     tlm_aligned(B, 16);
-  if (tiled) {
+  const bool tiled = vec && M > 16 && K < (1 << 23);
+  if (vec && gt::run_tiles<FMT == 0 ? gt::EL_E4M3 : gt::EL_E5M2, true, OUT>(A, B, C, M, N, K, s)) {
+    // tlm_gemm_tile.h: the shapes whose 256x256 tiles would not fill the chip
+  } else if (tiled) {
     const int64_t tiles = (int64_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
     gemm8_256x256<FMT, OUT><<<(unsigned)tiles, NTHREADS, 0, s>>>(
         (const uint8_t*)A, (const uint8_t*)B, C, M, N, K);
