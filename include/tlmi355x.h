@@ -120,6 +120,17 @@ int tlm_rope(const void* q, const void* k, const void* cos_t, const void* sin_t,
 int tlm_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int in_dtype,
              int out_dtype, int trans_b, void* stream);
 
+/* The gated half of the MLP programs (tpu_demo/ppl/mlp/mlp_bf16.py:98-131): H = up * silu(gate) with
+ * gate = A B_gate^T and up = A B_up^T, each rounded to dtype before the SwiGLU (fp32), as the programs'
+ * 16-bit tiles are: the result of two tlm_gemm calls and tlm_swiglu. A [M, K], B_gate, B_up [N, K],
+ * H [M, N], dtype F16 | BF16. One kernel where the tiles of both products do not fill the 256 x 256
+ * kernel (split K as tlm_gemm, never inside a stream capture); otherwise, or when A, B_gate or B_up is
+ * not 16-byte aligned, the three calls, for which tmp holds M N elements (else tmp may be NULL).
+ * tlm_gemm_swiglu_tmp_bytes: bytes of tmp that aligned operands of this shape need (0: none). */
+size_t tlm_gemm_swiglu_tmp_bytes(int64_t M, int64_t N, int64_t K);
+int tlm_gemm_swiglu(const void* A, const void* B_gate, const void* B_up, void* H, void* tmp,
+                    int64_t M, int64_t N, int64_t K, int dtype, void* stream);
+
 /* FP8 GEMM: C[M,N] = A[M,K] * B^T with B [N,K] row-major (trans_b == 1; trans_b == 0 takes B
  * [K,N] through a per-output fallback), fp32 accumulation, one rounding to out_dtype.
  * Reference: examples/gemm_fp8/example_tilelang_gemm_fp8.py:17-37 (T.gemm transpose_B=True,

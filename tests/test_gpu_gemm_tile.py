@@ -112,3 +112,21 @@ def test_gemm_split_tiles_repeat_and_replay():
         for c in outs:
             c.zero_()
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 72), (16, 2048, 1024), (33, 1000, 520), (64, 2048, 7168),
+                                   (100, 76, 256), (129, 1408, 2048), (520, 520, 264), (4, 64, 60),
+                                   (4096, 4096, 128)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_gemm_swiglu(M, N, K, dt):
+    """up * silu(gate) of two products, each rounded to the dtype first; K 60 and a weight that is not
+    16-byte aligned run as three calls. Three roundings of half an ulp each."""
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g, device=DEV).to(dt)
+    w = [(torch.randn(N * K + 1, generator=g, device=DEV) * K ** -0.5).to(dt) for _ in range(2)]
+    for shift in (0, 1) if M <= 33 else (0,):
+        bg, bu = (x[shift:shift + N * K].view(N, K) for x in w)
+        h = torch.full((M, N), float("nan"), dtype=dt, device=DEV)
+        ops.gemm_swiglu(a, bg, bu, h)
+        gate, up = a.double() @ bg.double().T, a.double() @ bu.double().T
+        assert _rel(h, up * gate * torch.sigmoid(gate)) < 3 * ULP[dt]

@@ -786,3 +786,52 @@ extern "C" int tlm_gemm(const void* A, const void* B, void* C, int64_t M, int64_
   return trans_b ? by_out<false, true>(A, B, C, m, n, k, out_dtype, s)
                  : by_out<false, false>(A, B, C, m, n, k, out_dtype, s);
 }
+
+extern "C" size_t tlm_gemm_swiglu_tmp_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K < 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return 0;
+  return gt::dual_plan(M, N, K).tile < 0 ? (size_t)M * N * 2 : 0;
+}
+
+extern "C" int tlm_gemm_swiglu(const void* A, const void* B_gate, const void* B_up, void* H,
+                               void* tmp, int64_t M, int64_t N, int64_t K, int dtype,
+                               void* stream) {
+  if (!A || !B_gate || !B_up || !H) {
+    tlm_set_error("tlm_gemm_swiglu: null pointer argument");
+    return TLM_EINVAL;
+  }
+  if (M < 0 || N < 0 || K < 0 || M > INT32_MAX || N > INT32_MAX / 2 || K > INT32_MAX ||
+      M * N > ((int64_t)1 << 39)) {
+    tlm_set_error("tlm_gemm_swiglu: bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N,
+                  (long long)K);
+    return TLM_EINVAL;
+  }
+  if (dtype != TLM_F16 && dtype != TLM_BF16) {
+    tlm_set_error("tlm_gemm_swiglu: dtype %d unsupported (F16 or BF16)", dtype);
+    return TLM_EUNSUPPORTED;
+  }
+  if (!tlm_aligned(A, 2) || !tlm_aligned(B_gate, 2) || !tlm_aligned(B_up, 2) || !tlm_aligned(H, 2)) {
+    tlm_set_error("tlm_gemm_swiglu: misaligned pointer");
+    return TLM_EINVAL;
+  }
+  if (M == 0 || N == 0) return TLM_OK;
+  hipStream_t s = (hipStream_t)stream;
+  if (tlm_aligned(A, 16) && tlm_aligned(B_gate, 16) && tlm_aligned(B_up, 16)) {
+    const gt::Plan p = gt::dual_plan(M, N, K);
+    if (p.tile >= 0) {
+      if (dtype == TLM_BF16)
+        gt::run_swiglu<gt::EL_BF16, TLM_BF16>(p, A, B_gate, B_up, H, (int)M, (int)N, (int)K, s);
+      else
+        gt::run_swiglu<gt::EL_F16, TLM_F16>(p, A, B_gate, B_up, H, (int)M, (int)N, (int)K, s);
+      TLM_LAUNCH_CHECK("tlm_gemm_swiglu");
+      return TLM_OK;
+    }
+  }
+  if (!tmp || !tlm_aligned(tmp, 2)) {
+    tlm_set_error("tlm_gemm_swiglu: these operands need a tmp of M N elements");
+    return TLM_EWORKSPACE;
+  }
+  int rc = tlm_gemm(A, B_gate, H, M, N, K, dtype, dtype, 1, stream);
+  if (rc == TLM_OK) rc = tlm_gemm(A, B_up, tmp, M, N, K, dtype, dtype, 1, stream);
+  if (rc == TLM_OK) rc = tlm_swiglu(H, tmp, H, M * N, dtype, stream);
+  return rc;
+}

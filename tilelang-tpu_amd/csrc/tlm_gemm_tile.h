@@ -43,7 +43,7 @@ constexpr uint32_t OOB_OFF = 0xfffffff0u;  // past num_records: the load returns
 constexpr int RSRC3 = 0x00020000;
 
 template <int EL_, bool TRANS_B_, int BM_, int BN_, int WTM_, int WTN_, int BKB_, int NST_,
-          bool NT_ = false, bool WIDE_ = false>
+          bool NT_ = false, bool WIDE_ = false, bool DUAL_ = false>
 struct Cfg {
   static constexpr int EL = EL_, BM = BM_, BN = BN_, WTM = WTM_, WTN = WTN_;
   static constexpr int BKB = BKB_;  // bytes of k per tile
@@ -51,6 +51,8 @@ struct Cfg {
   static constexpr int B_CP = NT_ ? CP_NT : CP_PLAIN;  // cache policy of B's loads
   static constexpr bool TRANS_B = TRANS_B_;
   static constexpr bool FP8 = EL >= EL_E4M3;
+  static constexpr bool DUAL = DUAL_;  // two B^T matrices, SwiGLU of the two products
+  static constexpr int BNC = DUAL ? BN / 2 : BN;  // columns of C
   static constexpr bool WIDE = WIDE_;  // fp8 operands multiplied as fp16
   static constexpr int ES = FP8 ? 1 : 2;
   static constexpr int BK = BKB / ES;
@@ -66,6 +68,7 @@ struct Cfg {
   static_assert(WM * WN * KG == 8 && SPG * KG == STEPS && QO * KG == Q, "wave layout");
   static_assert(NA * 8192 == SA && NB * 8192 == SB, "whole LDS-DMA instructions per wave");
   static_assert(!FP8 || TRANS_B, "fp8 takes B^T");
+  static_assert(!DUAL || (!FP8 && TRANS_B && NT % 2 == 0 && QO % 2 == 0), "pairs of column tiles");
   static constexpr int RED = KG > 1 ? 8 * Q * 1024 : 0;
   static constexpr int SMEM = NST * ST > RED ? NST * ST : RED;
   static_assert(SMEM <= 160 * 1024, "LDS");
@@ -147,7 +150,7 @@ TLM_DEV f32x16 mma8(u32x4 a0, u32x4 a1, u32x4 b0, u32x4 b1, f32x16 c) {
 }
 
 // The same product on the fp16 matrix instruction (every e4m3 / e5m2 value is an fp16 value): the fp8
-// one drops low bits of the sums (1.3e-5 of a K 4096 product against 4e-7 here).
+// one drops low bits of the sums (1.3e-5 of a K 4096 product against 3e-8 here).
 template <int EL>
 TLM_DEV f16x8 widen(uint32_t lo, uint32_t hi) {
   typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -230,7 +233,8 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_tile(const uint8_t* __restric
                                                        const uint8_t* __restrict__ B,
                                                        void* __restrict__ C, int M, int N, int K,
                                                        int ns, float* __restrict__ part,
-                                                       unsigned* __restrict__ arrivals) {
+                                                       unsigned* __restrict__ arrivals,
+                                                       const uint8_t* __restrict__ B2) {
   constexpr int BM = CF::BM, BN = CF::BN, BKB = CF::BKB, ES = CF::ES, KG = CF::KG;
   constexpr bool FP8 = CF::FP8, TRANS_B = CF::TRANS_B;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[CF::SMEM];
@@ -242,12 +246,12 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_tile(const uint8_t* __restric
   // Workgroup ids go round-robin over the 8 XCDs: XCD x takes a contiguous range of (split, column
   // tile, row tile), row tiles fastest, so that the row tiles that share a strip of B, and the
   // strips that share a k range of A, meet in one L2.
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + CF::BNC - 1) / CF::BNC;
   const int total = tiles_m * tiles_n * ns;
   const int xcd = blockIdx.x & 7, xi = blockIdx.x >> 3;
   const int lin = xcd * (total >> 3) + min(xcd, total & 7) + xi;
   const int tile = lin % (tiles_m * tiles_n), split = lin / (tiles_m * tiles_n);
-  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * CF::BNC;
   const int KT = (int)(((int64_t)K * ES + BKB - 1) / BKB);
   const int kt_lo = (int)((int64_t)split * KT / ns);
   const int n = (int)((int64_t)(split + 1) * KT / ns) - kt_lo;
@@ -263,8 +267,10 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_tile(const uint8_t* __restric
       constexpr int CPR = BKB / 16;
       const int r = ins * (64 / CPR) + lane / CPR;
       const int c = (lane % CPR) ^ swz_row<BKB>(r);
-      const bool ok = j < CF::NA ? m0 + r < M : n0 + r < N;
-      off[j] = ok ? (uint32_t)(r * K * ES + 16 * c) : OOB_OFF;
+      // DUAL: 16-row blocks of the tile alternate between the two matrices
+      const int rr = CF::DUAL && j >= CF::NA ? (r >> 5) * 16 + (r & 15) : r;
+      const bool ok = j < CF::NA ? m0 + rr < M : n0 + rr < N;
+      off[j] = ok ? (uint32_t)(rr * K * ES + 16 * c) : OOB_OFF;
       kch[j] = c * (16 / ES);
     } else {
       constexpr int CPR = BN * 2 / 16;
@@ -275,7 +281,10 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_tile(const uint8_t* __restric
     }
   }
   const uint8_t* const a_base = A + (int64_t)m0 * K * ES;
-  const uint8_t* const b_base = TRANS_B ? B + (int64_t)n0 * K * ES : B + (int64_t)n0 * 2;
+  // (a wave's instructions fill blocks of one of them: 8 instructions are whole pairs of blocks)
+  const bool second = CF::DUAL && (wave * (1024 / BKB) >> 4 & 1);
+  const uint8_t* const b_base =
+      TRANS_B ? (second ? B2 : B) + (int64_t)n0 * K * ES : B + (int64_t)n0 * 2;
   struct Fill {  // a tile's operand bases and LDS stage
     const uint8_t* a;
     const uint8_t* b;
@@ -546,6 +555,28 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_tile(const uint8_t* __restric
 
   // ---- C: the lane's quads are 4 consecutive columns of row m
   const bool vec_c = N % 4 == 0 && ((uintptr_t)C % (4 * out_size<OUT>())) == 0;
+  if constexpr (CF::DUAL) {
+    // column tiles nt, nt + 1 hold the same columns of the two products, rounded to the storage type as
+    // if stored, then up * gate / (1 + exp(-gate)) as tlm_swiglu
+    using H = h16<OUT == TLM_BF16>;
+    unroll<0, CF::Q / 2>([&](auto pc) __attribute__((always_inline)) {
+      constexpr int u = 2 * decltype(pc)::value, v = u % CF::QO;
+      if (kg == u / CF::QO) {
+        constexpr int mt = u / CF::NT, nt = u % CF::NT;
+        const int m = m0 + wm * CF::WTM + mt * CF::TR + lr;
+        const int c = n0 + (wn * CF::WTN + nt * CF::TR) / 2 + 4 * lq;
+        f32x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float g = H::to_f32(H::from_f32(fin[v][i]));
+          const float up = H::to_f32(H::from_f32(fin[v + 1][i]));
+          o[i] = up * (g * __builtin_amdgcn_rcpf(fast_exp(-g) + 1.0f));
+        }
+        if (m < M && c < N) store4<OUT>(C, (int64_t)m * N + c, o, min(4, N - c), vec_c);
+      }
+    });
+    return;
+  }
   unroll<0, CF::Q>([&](auto uc) __attribute__((always_inline)) {
     constexpr int u = decltype(uc)::value;
     if (kg == u / CF::QO) {
@@ -591,7 +622,9 @@ struct Plan {
 // coefficients are a fit to measured times of every tile and split at 355 shapes (M 1-4096,
 // N and K 512-57344); the choice was on average 1.1% (16-bit) and 1.6% (fp8) slower than the
 // best measured one. max_ns 1: no split.
-inline Plan choose(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, int max_ns) {
+// dual: both matrices of run_swiglu, N columns in all; only_tiles: not the 256 x 256 kernel.
+inline Plan choose(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, int max_ns,
+                   bool dual = false, bool only_tiles = false) {
   struct Cost {
     double a, b0, b1;  // launch; per k-tile alone; more per k-tile with every CU at work
   };
@@ -610,11 +643,13 @@ inline Plan choose(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, int 
   const Cost* const cost = fp8 ? C8 : C16;
   const bool only32 = fp8 && M <= 16;  // the one tile with an fp16 product
   Plan best{-1, 1};
-  double t_best = only32 ? 1e300 : run(cost[T_COUNT], tiles(256, 256), (kb + 127) / 128);
+  double t_best = only32 || only_tiles ? 1e300 : run(cost[T_COUNT], tiles(256, 256), (kb + 127) / 128);
+  if (dual) t_best += 10.0 + (double)M * (double)N * 3e-6 / 6.0;  // two more launches, SwiGLU's bytes
   for (int t = 0; t < T_COUNT; ++t) {
     if (only32 && t != T32) continue;
     if ((t == T32 || t == T32W) && M > 32) continue;
-    if (t == T32W && trans_b) continue;  // wider rows of row-major B only
+    // wider rows for row-major B; the pairs of column tiles of a dual product
+    if ((t == T32W && trans_b && !dual) || (t == T32 && dual)) continue;
     if ((t == T64N) != (M <= 64) && (t == T64N || t == T64)) continue;
     const Shape s = SHAPES[t];
     const int64_t tl = tiles(s.bm, s.bn), kt = (kb + s.bkb - 1) / s.bkb;
@@ -637,10 +672,21 @@ inline Plan choose(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, int 
 
 template <typename CF, int OUT>
 void launch_tile(const void* A, const void* B, void* C, int M, int N, int K, int ns, float* part,
-                 unsigned* arrivals, hipStream_t s) {
-  const int64_t wg = (int64_t)((M + CF::BM - 1) / CF::BM) * ((N + CF::BN - 1) / CF::BN) * ns;
+                 unsigned* arrivals, hipStream_t s, const uint8_t* B2 = nullptr) {
+  const int64_t wg = (int64_t)((M + CF::BM - 1) / CF::BM) * ((N + CF::BNC - 1) / CF::BNC) * ns;
   gemm_tile<CF, OUT><<<(unsigned)wg, THREADS, 0, s>>>((const uint8_t*)A, (const uint8_t*)B, C, M, N,
-                                                      K, ns, part, arrivals);
+                                                      K, ns, part, arrivals, B2);
+}
+
+// Whether a split may run on stream `s` (a 16-bit call with M <= 16 also inside a capture), and its
+// workspace.
+inline bool split_workspace(hipStream_t s, bool in_capture, float** part, unsigned** arrivals) {
+  if (s == hipStreamPerThread) return false;  // one handle for a stream of every thread
+  if (!in_capture) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
+  }
+  return tlm_split_slot(s, part, arrivals);
 }
 
 // Runs the plan's tile; false when the plan is the 256 x 256 kernel (or the shape does not fit the tiles'
@@ -656,14 +702,8 @@ bool run_tiles(const void* A, const void* B, void* C, int M, int N, int K, hipSt
   Plan p = choose(FP8, TB, M, N, K, 16);
   float* part = nullptr;
   unsigned* arrivals = nullptr;
-  if (p.ns > 1) {
-    bool ok = s != hipStreamPerThread;  // one handle for a stream of every thread
-    if (ok && (M > 16 || FP8)) {
-      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-      ok = hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
-    }
-    if (!ok || !tlm_split_slot(s, &part, &arrivals)) p = choose(FP8, TB, M, N, K, 1);
-  }
+  if (p.ns > 1 && !split_workspace(s, M <= 16 && !FP8, &part, &arrivals))
+    p = choose(FP8, TB, M, N, K, 1);
   switch (p.tile) {
     case T32:
       // 16 rows or fewer of fp8 are multiplied as fp16, which costs nothing beside B's stream and
@@ -685,6 +725,44 @@ bool run_tiles(const void* A, const void* B, void* C, int M, int N, int K, hipSt
     case T128: launch_tile<C128<EL, TB>, OUT>(A, B, C, M, N, K, p.ns, part, arrivals, s); return true;
     case T256: launch_tile<C256<EL, TB>, OUT>(A, B, C, M, N, K, p.ns, part, arrivals, s); return true;
     default: return false;
+  }
+}
+
+// ---- up * silu(gate) of two products with one A: gate = A B^T, up = A B2^T, both [M, N]. The MLP of
+// 64 tokens (7168 x 2048) spent its time in launches and their gaps: two products, SwiGLU (4.6 us for
+// 0.8 MB) and the down product took 46.5 us; with the first three in one kernel 27.3.
+inline Plan dual_plan(int64_t M, int64_t N, int64_t K) {
+  if (256 * K * 2 >= 0x7ffffff0 || K <= 0 || K % 8) return Plan{-1, 1};
+  return choose(false, true, M, 2 * N, K, 16, true);
+}
+template <int EL, int OUT>
+void run_swiglu(Plan p, const void* A, const void* B, const void* B2, void* C, int M, int N, int K,
+                hipStream_t s) {
+  float* part = nullptr;
+  unsigned* arrivals = nullptr;
+  if (p.ns > 1 && !split_workspace(s, false, &part, &arrivals))
+    p = choose(false, true, M, 2 * (int64_t)N, K, 1, true, true);
+  const uint8_t* const b2 = (const uint8_t*)B2;
+  switch (p.tile) {
+    case T32W:
+      launch_tile<Cfg<EL, true, 32, 128, 32, 64, 256, 3, true, false, true>, OUT>(
+          A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
+      break;
+    case T64N:
+      launch_tile<Cfg<EL, true, 64, 64, 32, 32, 256, 3, true, false, true>, OUT>(
+          A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
+      break;
+    case T64:
+      launch_tile<Cfg<EL, true, 64, 64, 32, 32, 256, 3, false, false, true>, OUT>(
+          A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
+      break;
+    case T128:
+      launch_tile<Cfg<EL, true, 128, 128, 64, 64, 128, 3, false, false, true>, OUT>(
+          A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
+      break;
+    default:
+      launch_tile<Cfg<EL, true, 256, 128, 64, 64, 128, 3, false, false, true>, OUT>(
+          A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
   }
 }
 

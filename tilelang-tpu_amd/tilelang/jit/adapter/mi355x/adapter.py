@@ -85,7 +85,7 @@ def _run_plan(plan, t: List[torch.Tensor], workspace_cache: dict):
         ops.flash_attn_fwd(t[a["q"]], t[a["k"]], t[a["v"]], t[a["o"]], a["causal"], a["sm_scale"],
                            operand_dtype=odt)
     elif f == "mlp":
-        # gate / up projections into 16-bit temporaries, SiLU(gate) * up, down projection
+        # SiLU(gate) * up of the two projections into a 16-bit temporary, down projection
         x, out = t[a["x"]], t[a["out"]]
         wg, wu, wd = t[a["wg"]], t[a["wu"]], t[a["wd"]]
         M, I = a["M"], a["inter"]
@@ -94,10 +94,7 @@ def _run_plan(plan, t: List[torch.Tensor], workspace_cache: dict):
             # 16-bit result of the down projection is copied to the fp32 output
             x, wg, wu, wd = (_cast_to(v, odt) for v in (x, wg, wu, wd))
         gate = torch.empty(M, I, dtype=x.dtype, device=x.device)
-        up = torch.empty_like(gate)
-        ops.gemm(x, wg, gate, True)
-        ops.gemm(x, wu, up, True)
-        ops.swiglu(gate, up, gate)
+        ops.gemm_swiglu(x, wg, wu, gate)
         if odt is None:
             ops.gemm(gate, wd, out, True)
         else:

@@ -151,6 +151,28 @@ def gemm(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, trans_b: bool = Fals
     return c
 
 
+def gemm_swiglu(a: torch.Tensor, b_gate: torch.Tensor, b_up: torch.Tensor, h: torch.Tensor):
+    """h = up * silu(gate), gate = a @ b_gate.T and up = a @ b_up.T rounded to the 16-bit dtype
+    (b_gate, b_up [N, K])."""
+    dev = _dev(a, b_gate, b_up, h)
+    for n, t in (("A", a), ("B_gate", b_gate), ("B_up", b_up), ("H", h)):
+        _contig(n, t)
+    M, K = a.shape
+    N = b_gate.shape[0]
+    if tuple(b_gate.shape) != (N, K) or tuple(b_up.shape) != (N, K) or tuple(h.shape) != (M, N):
+        raise ValueError(f"shape mismatch A{tuple(a.shape)} B_gate{tuple(b_gate.shape)} "
+                         f"B_up{tuple(b_up.shape)} H{tuple(h.shape)}")
+    if not (a.dtype == b_gate.dtype == b_up.dtype == h.dtype):
+        raise ValueError("A, B_gate, B_up and H must share a dtype")
+    ptrs = (a.data_ptr(), b_gate.data_ptr(), b_up.data_ptr())
+    tmp = None
+    if any(p & 15 for p in ptrs) or lib.load().tlm_gemm_swiglu_tmp_bytes(M, N, K):
+        tmp = torch.empty_like(h)
+    lib.call("tlm_gemm_swiglu", *ptrs, _ptr(h), _ptr(tmp), M, N, K, dtype_code(a.dtype),
+             _stream(dev))
+    return h
+
+
 def flash_attn_fwd(q, k, v, o, causal: bool, sm_scale: float,
                    operand_dtype: Optional[torch.dtype] = None):
     """BSHD attention forward: q, o [B, S, H, D]; k, v [B, S, H_kv, D] with H % H_kv == 0
