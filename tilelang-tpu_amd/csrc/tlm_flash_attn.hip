@@ -392,7 +392,8 @@ __global__ __launch_bounds__(64 * FA_WAVES, 1) void fa_fwd(const uint16_t* __res
 // Head dim 128: ping-pong kernel.
 //
 //   * workgroup = 8 waves = 256 queries of one (batch, head); a wave owns one 32-query block and
-//     computes S^T = K Q^T and O^T = V^T P^T with v_mfma_f32_16x16x32 (two 16-query tiles; Q^T
+//     computes S^T = K Q^T and O^T = V^T P^T with v_mfma_f32_16x16x32 (NQ = 2 16-query tiles, or one
+//     where 128-query workgroups finish earlier: fa_tiles; Q^T
 //     in VGPRs, P^T straight from the S^T accumulator). A lane holds 16 keys of each of its two
 //     queries, so the softmax statistics combine the four lane groups with xor-16 and xor-32
 //     exchanges. The 16x16 shape draws less power per FLOP than 32x32x16 (a higher sustained
@@ -422,7 +423,7 @@ __global__ __launch_bounds__(64 * FA_WAVES, 1) void fa_fwd(const uint16_t* __res
 //     tiles of a (batch, head) together, heaviest first: its K/V tiles are then read from that
 //     XCD's L2 by up to 16 workgroups at about the same time.
 constexpr int PP_D = 128;
-constexpr int PP_BQ = 256;                        // queries per workgroup
+constexpr int PP_BQ = 256;                        // queries per workgroup (128 with one query tile per wave)
 constexpr int PP_KV = 64;                         // keys per tile
 constexpr int PP_TILE = PP_KV * PP_D * 2;         // bytes of one K or V tile
 constexpr int PP_NST = 4;                         // ring stages (tiles j-1 .. j+2 live in step j)
@@ -494,16 +495,19 @@ TLM_DEV void phase_barrier() {
 }
 
 // NT (split parts whose K / V tiles are each read by one workgroup): non-temporal K / V loads.
-template <bool BF16, bool CAUSAL, bool OUT32, bool SPLIT = false, bool NT = false>
+template <bool BF16, bool CAUSAL, bool OUT32, bool SPLIT = false, bool NT = false, int NQ = 2>
 __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__ Q,
                                                    const uint16_t* __restrict__ K,
                                                    const uint16_t* __restrict__ V,
                                                    void* __restrict__ O, int B, int S, int H,
-                                                   int Hkv, float sc, SeqMap sm, FaSplit sp) {
+                                                   int Hkv, float sc, SeqMap sm, FaSplit sp,
+                                                   int pairs) {
   static_assert(!SPLIT || (OUT32 && !CAUSAL), "split parts are non-causal with fp32 output");
   using MT = fa_mma16<BF16>;
   using v8 = typename MT::v8;
   using HH = h16<BF16>;
+  constexpr int WQ = 16 * NQ;       // queries per wave
+  constexpr int TQ = 8 * WQ;        // queries per tile
   __shared__ __attribute__((aligned(1024))) uint8_t smem[PP_SMEM];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -522,8 +526,8 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
   // workgroup carries the same work. The dispatcher gives every CU the same number of workgroups
   // whatever their length (measured: 16 per CU at B 8, H 32, S 4096), so workgroups of unequal
   // work leave CUs idle; one tile per workgroup kept them busy 79% of the time.
-  const int nqt = (S + PP_BQ - 1) / PP_BQ;
-  const int nslot = CAUSAL ? (nqt + 1) / 2 : nqt;
+  const int nqt = (S + TQ - 1) / TQ;
+  const int nslot = CAUSAL && pairs ? (nqt + 1) / 2 : nqt;
   const int G = H / Hkv;
   int lin = blockIdx.x;
   int b, h, slot, si = 0;
@@ -535,9 +539,10 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
     const int xcd = lin & 7, s = lin >> 3;
     const int per = nslot * G;  // workgroups per K/V head
     const int kvh = (s / per) * 8 + xcd, rem = s % per;
-    slot = rem % nslot;
+    // single tiles: the longest tiles of every head first
+    slot = CAUSAL && !pairs ? rem / G : rem % nslot;
     b = kvh / Hkv;
-    h = (kvh % Hkv) * G + rem / nslot;
+    h = (kvh % Hkv) * G + (CAUSAL && !pairs ? rem % G : rem / nslot);
   } else {
     const int bh = lin / nslot;
     slot = lin % nslot;
@@ -548,11 +553,11 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
   // Causal: query i sees keys j <= i + (Sk - Sq) (bottom-right aligned; 0 offset when dense).
   SeqRange sr = seq_range(sm, b);
   if constexpr (SPLIT) sr = split_keys(sr, sp, si);
-  const int n_items = CAUSAL && 2 * slot != nqt - 1 ? 2 : 1;
+  const int n_items = CAUSAL && pairs && 2 * slot != nqt - 1 ? 2 : 1;
   for (int item = 0; item < n_items; ++item) {
   const int qt = CAUSAL && item == 0 ? nqt - 1 - slot : slot;
   [&]() TLM_INLINE {  // one query tile; a return ends the tile
-  const int q0 = qt * PP_BQ;
+  const int q0 = qt * TQ;
   const int Sq = sr.nq, Sk = sr.nk, coff = Sk - Sq;
   if (q0 >= Sq) return;  // whole workgroup
   const int64_t rs = sm.tq;     // elements between consecutive tokens of Q, O
@@ -562,22 +567,24 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
   const uint16_t* Qb = Q + head;
 
   const int n_all = (Sk + PP_KV - 1) / PP_KV;
-  const int kv_vis = q0 + PP_BQ + coff;  // keys visible to the workgroup's last query row, + 1
+  const int kv_vis = q0 + TQ + coff;  // keys visible to the workgroup's last query row, + 1
   const int n = CAUSAL ? (kv_vis <= 0 ? 0 : min(n_all, (kv_vis + PP_KV - 1) / PP_KV))
                        : n_all;  // key tiles of the workgroup
-  const int qb0 = q0 + 32 * blk;  // first query of the wave
-  const int w_last = qb0 + 31 + coff;  // last key visible to the wave
+  const int qb0 = q0 + WQ * blk;  // first query of the wave
+  const int w_last = qb0 + WQ - 1 + coff;  // last key visible to the wave
   const int nw = qb0 >= Sq ? 0 : (CAUSAL ? (w_last < 0 ? 0 : min(n, w_last / PP_KV + 1)) : n);
 
   // v_mfma_f32_16x16x32 roles: lane l works on column (query) l % 16 of a 16-wide tile and on
-  // k group g = l / 16; the wave's 32 queries are two 16-query tiles qq
+  // k group g = l / 16; the wave's queries are NQ 16-query tiles qq
   const int ql = lane & 15, g = lane >> 4;
-  const int my_q[2] = {qb0 + ql, qb0 + 16 + ql};
+  int my_q[NQ];
+#pragma unroll
+  for (int qq = 0; qq < NQ; ++qq) my_q[qq] = qb0 + 16 * qq + ql;
 
   // Q^T operand (B of S^T = K Q^T): lane holds query my_q[qq], d = 32 dk + 8 g .. + 7
-  v8 qreg[2][PP_D / 32];
+  v8 qreg[NQ][PP_D / 32];
 #pragma unroll
-  for (int qq = 0; qq < 2; ++qq)
+  for (int qq = 0; qq < NQ; ++qq)
 #pragma unroll
     for (int dk = 0; dk < PP_D / 32; ++dk) {
       u32x4 v = {0, 0, 0, 0};
@@ -632,12 +639,16 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
     vaddr[dt] = sbase + PP_VRING + (uint32_t)(vrow * 256 + 16 * c + 8 * (jj & 1));
   }
 
-  f32x4 oacc[PP_D / 16][2];  // O^T: [16-dim tile][query tile], element i = dim 16 dt + 4 g + i
+  f32x4 oacc[PP_D / 16][NQ];  // O^T: [16-dim tile][query tile], element i = dim 16 dt + 4 g + i
 #pragma unroll
-  for (int t = 0; t < PP_D / 16; ++t) oacc[t][0] = oacc[t][1] = f32x4{};
-  f32x4 sacc[4][2];  // S^T: [16-key tile][query tile], element i = key 16 kt + 4 g + i
-  u32x4 pb[2][2];    // P^T operands of the last softmax: [32-key step][query tile]
-  float m_run[2] = {-INFINITY, -INFINITY}, l_part[2] = {0.f, 0.f};
+  for (int t = 0; t < PP_D / 16; ++t)
+#pragma unroll
+    for (int qq = 0; qq < NQ; ++qq) oacc[t][qq] = f32x4{};
+  f32x4 sacc[4][NQ];  // S^T: [16-key tile][query tile], element i = key 16 kt + 4 g + i
+  u32x4 pb[2][NQ];   // P^T operands of the last softmax: [32-key step][query tile]
+  float m_run[NQ], l_part[NQ];
+#pragma unroll
+  for (int qq = 0; qq < NQ; ++qq) m_run[qq] = -INFINITY, l_part[qq] = 0.f;
 
   // ---- MFMA phase: QK of the tile in the current K stage (16 operands x 2 query tiles), then
   // PV of the tile in the current V stage (16 operands x 2 query tiles). Operand reads run DEPTH
@@ -680,12 +691,12 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
       if constexpr (m < NQK) {
         constexpr int dk = m / 4, kt = m % 4;
 #pragma unroll
-        for (int qq = 0; qq < 2; ++qq)
+        for (int qq = 0; qq < NQ; ++qq)
           sacc[kt][qq] = MT::mma(a, qreg[qq][dk], dk == 0 ? f32x4{} : sacc[kt][qq]);
       } else {
         constexpr int mm = m - NQK, ks = mm / 8, dt = mm % 8;
 #pragma unroll
-        for (int qq = 0; qq < 2; ++qq)
+        for (int qq = 0; qq < NQ; ++qq)
           oacc[dt][qq] = MT::mma(a, __builtin_bit_cast(v8, pb[ks][qq]), oacc[dt][qq]);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -722,19 +733,19 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
         for (int i = 0; i < 4; ++i) {
           const int key = k0 + 16 * kt + 4 * g + i;
 #pragma unroll
-          for (int qq = 0; qq < 2; ++qq)
+          for (int qq = 0; qq < NQ; ++qq)
             if (key >= Sk || (CAUSAL && key > my_q[qq] + coff)) sacc[kt][qq][i] = -INFINITY;
         }
     }
     // the first tile (m = -inf) always needs its max: skip the exponentials it would redo
-    float ts[2] = {0.f, 0.f};
+    float ts[NQ] = {};
     if (j > 0) {
-      ts[0] = exp_tile(0, -m_run[0]);
-      ts[1] = exp_tile(1, -m_run[1]);
-    }
-    if (j == 0 || __builtin_amdgcn_ballot_w64(!(ts[0] <= P_LIMIT) || !(ts[1] <= P_LIMIT))) {
 #pragma unroll
-      for (int qq = 0; qq < 2; ++qq) {
+      for (int qq = 0; qq < NQ; ++qq) ts[qq] = exp_tile(qq, -m_run[qq]);
+    }
+    if (j == 0 || __builtin_amdgcn_ballot_w64(!(ts[0] <= P_LIMIT) || !(ts[NQ - 1] <= P_LIMIT))) {
+#pragma unroll
+      for (int qq = 0; qq < NQ; ++qq) {
         float mx = -INFINITY;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
@@ -751,8 +762,8 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
         ts[qq] = exp_tile(qq, m_new == -INFINITY ? 0.f : -m_new);
       }
     }
-    l_part[0] += ts[0];
-    l_part[1] += ts[1];
+#pragma unroll
+    for (int qq = 0; qq < NQ; ++qq) l_part[qq] += ts[qq];
   };
 
   // ---- schedule. Step j: group 0 runs X(j) = QK(j) + PV(j-1), then Y(j) = softmax(j); group 1
@@ -821,9 +832,9 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
 
   // ---- epilogue: lane holds O^T[d = 16 dt + 4 g + i][query my_q[qq]]; the row sums of a query
   // are spread over the four lane groups
-  float inv[2], l_all[2];
+  float inv[NQ], l_all[NQ];
 #pragma unroll
-  for (int qq = 0; qq < 2; ++qq) {
+  for (int qq = 0; qq < NQ; ++qq) {
     float l_tot = l_part[qq] + __shfl_xor(l_part[qq], 16, 64);
     l_tot += __shfl_xor(l_tot, 32, 64);
     l_all[qq] = l_tot;
@@ -837,7 +848,7 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
     }
     float* Of = (float*)O + ob;
 #pragma unroll
-    for (int qq = 0; qq < 2; ++qq)
+    for (int qq = 0; qq < NQ; ++qq)
       if (my_q[qq] < Sq) {
 #pragma unroll
         for (int dt = 0; dt < PP_D / 16; ++dt)
@@ -850,9 +861,9 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
       }
     return;
   }
-  uint16_t* stage = (uint16_t*)smem + wave * 32 * PP_OP;  // [32 queries][PP_OP]
+  uint16_t* stage = (uint16_t*)smem + wave * WQ * PP_OP;  // [WQ queries][PP_OP]
 #pragma unroll
-  for (int qq = 0; qq < 2; ++qq)
+  for (int qq = 0; qq < NQ; ++qq)
 #pragma unroll
     for (int dt = 0; dt < PP_D / 16; ++dt) {
       const f32x4 o = oacc[dt][qq] * inv[qq];
@@ -864,7 +875,7 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   uint16_t* Ob = (uint16_t*)O + head;
 #pragma unroll
-  for (int it = 0; it < 32 * (PP_D / 8) / 64; ++it) {
+  for (int it = 0; it < WQ * (PP_D / 8) / 64; ++it) {
     const int idx = lane + 64 * it;
     const int r = idx / (PP_D / 8), c = (idx % (PP_D / 8)) * 8;
     const int q = qb0 + r;
@@ -876,20 +887,73 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
   }
 }
 
-template <bool BF16, bool CAUSAL, bool OUT32, bool SPLIT = false, bool NT = false>
-int launch_pp(const void* q, const void* k, const void* v, void* o, int B, int S, int H, int Hkv,
-              float sc, const SeqMap& sm, hipStream_t st, const FaSplit& sp = FaSplit{}) {
-  const int64_t nqt = (S + PP_BQ - 1) / PP_BQ;
-  // causal: two tiles per workgroup; split: one workgroup per internal key split
-  const int64_t nwg = (CAUSAL ? (nqt + 1) / 2 : nqt) * B * H * (SPLIT ? sp.nsi : 1);
+// Query tiles per wave (2: 256-query workgroups, 1: 128-query ones) and, for causal attention,
+// whether a workgroup takes a pair of tiles or one. Both kinds hold 128 KB of LDS, one workgroup per
+// CU. A step (64 keys) takes about 1.8 us with two query tiles per wave and 1.18 with one, and a tile
+// about 3 more steps to start and end: 256 queries are cheaper per query, and 128 win where the
+// larger tiles leave CUs idle or one CU with a long chain. Single causal tiles (longest first) end when the
+// longest one or the average CU does, 10% late for their unequal lengths. Measured (us, H 32, 8 K/V heads, causal;
+// 256 queries in pairs / 128 in pairs / 128 single): S 512 33.3 / 18.8 / 13.9, S 1111
+// 52.3 / 30.0 / 25.3, S 2048 72.4 / 49.6 / 48.7, S 4000 132 / 158 / 157; full attention, S 512
+// 17.7 (256) / 13.0 (128), S 1111 33.3 / 44.0.
+// `keys`: of the longest sequence; shorter ones of a ragged batch do not change which is longer.
+struct FaTiles {
+  int nq;
+  bool pairs;
+};
+FaTiles fa_tiles(bool causal, int64_t heads, int64_t S, int64_t keys) {
+  const double kt = (double)((keys + PP_KV - 1) / PP_KV);
+  const double off = keys > S ? (double)((keys - S) / PP_KV) : 0.0;  // keys before the first query
+  FaTiles best{2, true};
+  double t_best = 1e300;
+  auto take = [&](int nq, bool pairs, double t) {
+    if (t < t_best) t_best = t, best = FaTiles{nq, pairs};
+  };
+  for (int nq = 2; nq >= 1; --nq) {
+    const int64_t nqt = (S + 128 * nq - 1) / (128 * nq);
+    const double step = nq == 2 ? 1.8 : 1.18, nt = (double)nqt;
+    if (!causal) {
+      take(nq, true, step * (double)((nqt * heads + 255) / 256) * (kt + 3.0));
+      continue;
+    }
+    const double pair = nqt == 1 ? kt + 3.0 : 2.0 * off + 2.0 * nq * (nt + 1.0) + 6.0;
+    take(nq, true, step * (double)(((nqt + 1) / 2 * heads + 255) / 256) * pair);
+    if (nq == 1) {
+      const double all = (double)heads * nt * (off + nt + 1.0 + 3.0);
+      take(nq, false, step * std::max(kt + 3.0, 1.1 * all / 256.0));
+    }
+  }
+  return best;
+}
+
+template <bool BF16, bool CAUSAL, bool OUT32, bool SPLIT, bool NT, int NQ>
+int launch_pp_nq(const void* q, const void* k, const void* v, void* o, int B, int S, int H, int Hkv,
+                 float sc, const SeqMap& sm, hipStream_t st, const FaSplit& sp, bool pairs) {
+  const int64_t nqt = (S + 128 * NQ - 1) / (128 * NQ);
+  // causal pairs: two tiles per workgroup; split: one workgroup per internal key split
+  const int64_t nwg = (CAUSAL && pairs ? (nqt + 1) / 2 : nqt) * B * H * (SPLIT ? sp.nsi : 1);
   if (nwg > INT32_MAX) {
     tlm_set_error("tlm_flash_attn_fwd: problem too large");
     return TLM_EINVAL;
   }
-  fa_fwd_pp<BF16, CAUSAL, OUT32, SPLIT, NT><<<(unsigned)nwg, 512, 0, st>>>(
-      (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, o, B, S, H, Hkv, sc, sm, sp);
+  fa_fwd_pp<BF16, CAUSAL, OUT32, SPLIT, NT, NQ><<<(unsigned)nwg, 512, 0, st>>>(
+      (const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, o, B, S, H, Hkv, sc, sm, sp,
+      pairs ? 1 : 0);
   TLM_LAUNCH_CHECK("tlm_flash_attn_fwd");
   return TLM_OK;
+}
+
+template <bool BF16, bool CAUSAL, bool OUT32, bool SPLIT = false, bool NT = false>
+int launch_pp(const void* q, const void* k, const void* v, void* o, int B, int S, int H, int Hkv,
+              float sc, const SeqMap& sm, hipStream_t st, const FaSplit& sp = FaSplit{}) {
+  const int64_t heads = (int64_t)B * H * (SPLIT ? sp.nsi : 1);
+  const int64_t keys = SPLIT ? sp.per_i : sm.cu_q ? S : sm.s_k;
+  const FaTiles t = fa_tiles(CAUSAL, heads, S, keys);
+  if (t.nq == 2 || (NT && S > 128))  // NT: a K / V tile is read by one workgroup
+    return launch_pp_nq<BF16, CAUSAL, OUT32, SPLIT, NT, 2>(q, k, v, o, B, S, H, Hkv, sc, sm, st, sp,
+                                                           t.pairs);
+  return launch_pp_nq<BF16, CAUSAL, OUT32, SPLIT, NT, 1>(q, k, v, o, B, S, H, Hkv, sc, sm, st, sp,
+                                                         t.pairs);
 }
 
 template <bool BF16, bool CAUSAL, int D>
