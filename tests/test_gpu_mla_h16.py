@@ -1,0 +1,87 @@
+"""GPU parity of the balanced MLA decode over a 16-bit cache: sequences shorter and longer than a 64-token tile,
+empty ones, several ranges per sequence and several sequences per range, page sizes on both sides of a tile,
+head blocks, workspaces that hold few slots, and score jumps that move the reference maximum.
+
+Reference: fp64 attention over the gathered rows. Tolerance: P is rounded to the 16-bit type (2^-9
+bf16, 2^-12 fp16 relative per weight) and the output once: 2-norm error within two such ulps.
+"""
+import pytest
+import torch
+
+from tilelang.jit.adapter.mi355x import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+DV, DPE = 512, 64
+
+
+def _case(lens, H, page, dt, seed=0, ns=4, fused=True, jump=None, bad_page=False):
+    g = torch.Generator(device=DEV).manual_seed(seed + sum(lens) + H)
+    B = len(lens)
+    pages = max(1, -(-max(lens) // page))
+    rows = torch.randn(B * pages * page, DV + DPE, generator=g, device=DEV).to(dt)
+    if jump is not None:  # a few tokens far above the rest
+        rows[jump::97] *= 8
+    table = torch.randperm(B * pages, generator=g, device=DEV).view(B, pages).to(torch.int32)
+    sl = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    q = torch.randn(B, H, DV + DPE, generator=g, device=DEV).to(dt)
+    scale = (DV + DPE) ** -0.5
+    at = torch.arange(pages * page, device=DEV)
+    exp = torch.zeros(B, H, DV, dtype=torch.float64, device=DEV)
+    if bad_page:
+        table[0, 0] = B * pages + 7
+    for b, n in enumerate(lens):
+        if n:
+            row = table[b].long()[at[:n] // page] * page + at[:n] % page
+            ok = row < rows.shape[0]
+            kv = rows[row * ok].double() * ok[:, None]
+            exp[b] = torch.softmax(q[b].double() @ kv.T * scale, 1) @ kv[:, :DV]
+    kv, kpe = rows[:, :DV], rows[:, DV:]
+    if not fused:
+        kv, kpe = kv.contiguous(), kpe.contiguous()
+    out = torch.full((B, H, DV), float("nan"), dtype=dt, device=DEV)
+    ws = torch.empty(ops.mla_workspace_bytes(B, H, DV, ns), dtype=torch.uint8, device=DEV)
+    ops.mla_decode(q[..., :DV], q[..., DV:], kv, kpe, table, sl, out, ws, page, ns, scale)
+    return out, exp
+
+
+def _check(out, exp, lens, dt):
+    tol = 2 * (2.0 ** -9 if dt == torch.bfloat16 else 2.0 ** -12)
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert torch.equal(out[b], torch.zeros_like(out[b]))
+        else:
+            assert float((out[b].double() - exp[b]).norm() / exp[b].norm()) < tol, (b, n)
+
+
+@pytest.mark.parametrize("lens", [[1], [64], [65, 0, 63], [3000], [500, 4000, 1, 128, 0, 2000, 77, 640],
+                                  [33] * 40, [0, 0, 5], [1300] * 16])
+@pytest.mark.parametrize("H,page,dt", [(128, 64, torch.bfloat16), (64, 16, torch.float16),
+                                       (192, 100, torch.bfloat16), (256, 128, torch.float16)])
+def test_lengths_and_heads(lens, H, page, dt):
+    out, exp = _case(lens, H, page, dt)
+    _check(out, exp, lens, dt)
+
+
+@pytest.mark.parametrize("ns", [1, 2, 16, 64])
+@pytest.mark.parametrize("lens", [[700, 90, 2000], [900], [300] * 20])
+def test_workspace_sizes(ns, lens):
+    """num_split only sizes the workspace, and with it the number of ranges: fewer and more than sequences."""
+    for dt in (torch.bfloat16, torch.float16):
+        out, exp = _case(lens, 128, 64, dt, ns=ns, fused=False)
+        _check(out, exp, lens, dt)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_score_jumps(dt):
+    """Tiles far above the reference maximum (fp16: beyond 2^15 times it) go through the rescale."""
+    lens = [1000, 64, 300]
+    for jump in (0, 50, 96):
+        out, exp = _case(lens, 128, 64, dt, jump=jump, ns=2)
+        _check(out, exp, lens, dt)
+
+
+def test_rows_outside_the_pool_read_as_zeros():
+    lens = [200, 150]
+    out, exp = _case(lens, 128, 64, torch.bfloat16, bad_page=True)
+    _check(out, exp, lens, torch.bfloat16)
