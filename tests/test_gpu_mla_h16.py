@@ -85,3 +85,12 @@ def test_rows_outside_the_pool_read_as_zeros():
     lens = [200, 150]
     out, exp = _case(lens, 128, 64, torch.bfloat16, bad_page=True)
     _check(out, exp, lens, torch.bfloat16)
+
+
+@pytest.mark.parametrize("B,H", [(65, 128), (300, 192), (1100, 64)])
+def test_large_batches(B, H):
+    """The combine takes several heads per wave; empty, whole and cut sequences among them."""
+    lens = [(37 * b) % 90 for b in range(B)]
+    lens[B // 2] = 1500
+    out, exp = _case(lens, H, 16, torch.bfloat16, ns=1)
+    _check(out, exp, lens, torch.bfloat16)

@@ -5,7 +5,7 @@
 // heads a multiple of 64.
 //
 // What bounds it: fixed costs at small batches, the tile's own chain at large ones. 8 sequences of
-// 500 .. 4,000 tokens, 128 heads (bf16): 25.3 us and 8.5 us for the combine, where the split kernel that
+// 500 .. 4,000 tokens, 128 heads (bf16): 25.0 us and 8.0 us for the combine, where the split kernel that
 // it replaced took 67.2 and 14.7; 20.7 MB of cache rows would take 3.1 us. Inside a workgroup 1.6 us go to the
 // scan, 5 to the block table and Q, 2.6 to the first tile and 2 to 4 to the partial rows (33 MB of fp32 for
 // 128 ranges, written and read again); the rest is the launch. 16 x 4,000 .. 8,000 tokens: 61 us, of which a
@@ -549,73 +549,85 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
 }
 
 // Merge of the pieces of every sequence that no range holds whole, and zero rows for empty sequences. A wave
-// per head, 8 dims per lane; MH_BATCH pieces' rows requested together.
-constexpr int MH_CW = 4;  // heads per workgroup
+// per head and step, 8 dims per lane; MH_BATCH pieces' rows requested together. Bound by the partial rows
+// (4 to 5 TB/s of 33 MB) after two dependent loads. Every workgroup scans the lengths, so a large batch has
+// few per sequence: with one for every 4 heads, 4,096 sequences of 16 tokens took 1,307 us in all (now
+// 413; the split kernel 1,102). Two waves a workgroup instead of four: 8.2 -> 8.0 us at 8 x 500 .. 4,000
+// tokens, 11.0 -> 9.1 at 1 x 2,000.
+constexpr int MH_CW = 2;  // waves per workgroup
+constexpr int MH_CWGS = 4096;  // workgroups wanted
 constexpr int MH_BATCH = 8;
 template <bool O_BF16>
 __global__ __launch_bounds__(64 * MH_CW) void mla_h16_combine(const MhArgs a) {
   __shared__ int sh[MH_CW + 2];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int hblocks = a.Hq / MH_CW;
-  const int b = blockIdx.x / hblocks, head = blockIdx.x % hblocks * MH_CW + wave;
+  const int per_seq = gridDim.x / a.B, b = blockIdx.x / per_seq;
+  const int head0 = blockIdx.x % per_seq * MH_CW + wave, step = per_seq * MH_CW;
   const int tiles = mh_tiles(a, b);
   using HO = h16<O_BF16>;
-  uint16_t* const out = a.out + ((int64_t)b * a.Hq + head) * MH_DV + 8 * lane;
-  const MhPoint pt = mh_scan<64 * MH_CW, true>(a, sh, [&](int) { return b; });
+  uint16_t* const out_b = a.out + (int64_t)b * a.Hq * MH_DV + 8 * lane;
   if (tiles == 0) {
-    *(u32x2*)out = u32x2{0, 0};
-    *(u32x2*)(out + 4) = u32x2{0, 0};
+    for (int head = head0; head < a.Hq; head += step) {
+      uint16_t* const out = out_b + (int64_t)head * MH_DV;
+      *(u32x2*)out = u32x2{0, 0};
+      *(u32x2*)(out + 4) = u32x2{0, 0};
+    }
     return;
   }
+  const MhPoint pt = mh_scan<64 * MH_CW, true>(a, sh, [&](int) { return b; });
   const int ng = min(a.G, pt.total), x0 = pt.before + MH_PIECE;
   const int r0 = mh_range_of(pt.total, ng, x0), r1 = mh_range_of(pt.total, ng, x0 + tiles - 1);
   if (r0 == r1) return;  // written whole
   const int np = r1 - r0 + 1;
-  float mx = -INFINITY, sum = 0.f;
-  f32x4 acc[2] = {f32x4{}, f32x4{}};
-  for (int p0 = 0; p0 < np; p0 += MH_BATCH) {
-    f32x4 v[MH_BATCH][2];
-    float ls[MH_BATCH], top = mx;
+  for (int head = head0; head < a.Hq; head += step) {
+    uint16_t* const out = out_b + (int64_t)head * MH_DV;
+    float mx = -INFINITY, sum = 0.f;
+    f32x4 acc[2] = {f32x4{}, f32x4{}};
+    for (int p0 = 0; p0 < np; p0 += MH_BATCH) {
+      f32x4 v[MH_BATCH][2];
+      float ls[MH_BATCH], top = mx;
 #pragma unroll
-    for (int i = 0; i < MH_BATCH; ++i) {
-      ls[i] = -INFINITY;
-      v[i][0] = v[i][1] = f32x4{};
-      if (p0 + i < np) {
-        const int p = p0 + i;
-        const int64_t s = (int64_t)(p == 0 ? mh_head_slot(a, r0, b) : mh_tail_slot(r0 + p)) * a.Hq + head;
-        ls[i] = a.ws_lse[s];
-        const float* const o = a.ws_o + s * MH_DV + 8 * lane;
-        v[i][0] = *(const f32x4*)o;
-        v[i][1] = *(const f32x4*)(o + 4);
+      for (int i = 0; i < MH_BATCH; ++i) {
+        ls[i] = -INFINITY;
+        v[i][0] = v[i][1] = f32x4{};
+        if (p0 + i < np) {
+          const int p = p0 + i;
+          const int64_t s = (int64_t)(p == 0 ? mh_head_slot(a, r0, b) : mh_tail_slot(r0 + p)) * a.Hq + head;
+          ls[i] = a.ws_lse[s];
+          const float* const o = a.ws_o + s * MH_DV + 8 * lane;
+          v[i][0] = *(const f32x4*)o;
+          v[i][1] = *(const f32x4*)(o + 4);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < MH_BATCH; ++i) top = fmaxf(top, ls[i]);
+      const float al = mx == -INFINITY ? 0.f : fast_exp2(mx - top);
+      mx = top;
+      sum *= al;
+      acc[0] *= al;
+      acc[1] *= al;
+#pragma unroll
+      for (int i = 0; i < MH_BATCH; ++i) {
+        const float wt = ls[i] == -INFINITY ? 0.f : fast_exp2(ls[i] - mx);
+        sum += wt;
+        acc[0] += v[i][0] * wt;
+        acc[1] += v[i][1] * wt;
       }
     }
-#pragma unroll
-    for (int i = 0; i < MH_BATCH; ++i) top = fmaxf(top, ls[i]);
-    const float al = mx == -INFINITY ? 0.f : fast_exp2(mx - top);
-    mx = top;
-    sum *= al;
-    acc[0] *= al;
-    acc[1] *= al;
-#pragma unroll
-    for (int i = 0; i < MH_BATCH; ++i) {
-      const float wt = ls[i] == -INFINITY ? 0.f : fast_exp2(ls[i] - mx);
-      sum += wt;
-      acc[0] += v[i][0] * wt;
-      acc[1] += v[i][1] * wt;
-    }
+    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+    acc[0] *= inv;
+    acc[1] *= inv;
+    *(u32x2*)out = u32x2{HO::pack(acc[0][0], acc[0][1]), HO::pack(acc[0][2], acc[0][3])};
+    *(u32x2*)(out + 4) = u32x2{HO::pack(acc[1][0], acc[1][1]), HO::pack(acc[1][2], acc[1][3])};
   }
-  const float inv = sum > 0.f ? 1.0f / sum : 0.f;
-  acc[0] *= inv;
-  acc[1] *= inv;
-  *(u32x2*)out = u32x2{HO::pack(acc[0][0], acc[0][1]), HO::pack(acc[0][2], acc[0][3])};
-  *(u32x2*)(out + 4) = u32x2{HO::pack(acc[1][0], acc[1][1]), HO::pack(acc[1][2], acc[1][3])};
 }
 
 template <bool BF16, bool O_BF16>
 int mh_launch(const MhArgs& a, hipStream_t st) {
   mla_h16_decode<BF16, O_BF16><<<(unsigned)(a.G * (a.Hq / MH_HEADS)), 512, 0, st>>>(a);
   TLM_LAUNCH_CHECK("tlm_mla_decode (16-bit)");
-  mla_h16_combine<O_BF16><<<(unsigned)((int64_t)a.B * a.Hq / MH_CW), 64 * MH_CW, 0, st>>>(a);
+  const int per_seq = std::max(1, std::min(MH_CWGS / a.B, a.Hq / MH_CW));
+  mla_h16_combine<O_BF16><<<(unsigned)(a.B * per_seq), 64 * MH_CW, 0, st>>>(a);
   TLM_LAUNCH_CHECK("tlm_mla_decode (16-bit combine)");
   return TLM_OK;
 }
