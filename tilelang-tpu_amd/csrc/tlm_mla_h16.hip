@@ -33,7 +33,7 @@
 //     rows 8 tokens per instruction). The cache rows of 512 tokens at a time are looked up half a block
 //     ahead into an LDS table. 16-byte chunk c of token r sits at c ^ f(r), f(r) = 2 (r % 8) + r / 8 % 2:
 //     16 tokens' reads of one chunk column (S^T) and the transposed reads of 8 tokens x 2 chunks (V^T)
-////     both fall on all banks.
+//     both fall on all banks.
 #include "tlm_common.h"
 
 #include <algorithm>
