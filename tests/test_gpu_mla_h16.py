@@ -1,6 +1,6 @@
-"""GPU parity of the balanced MLA decode over a 16-bit cache: sequences shorter and longer than a 64-token tile,
+"""GPU parity of the balanced MLA decode over a 16-bit cache: sequences shorter and longer than a 32-token tile,
 empty ones, several ranges per sequence and several sequences per range, page sizes on both sides of a tile,
-head blocks, workspaces that hold few slots, and score jumps that move the reference maximum.
+head blocks, workspaces that hold few slots, scores of -inf, and score jumps that move the running maximum.
 
 Reference: fp64 attention over the gathered rows. Tolerance: P is rounded to the 16-bit type (2^-9
 bf16, 2^-12 fp16 relative per weight) and the output once: 2-norm error within two such ulps.
@@ -15,7 +15,7 @@ DEV = "cuda"
 DV, DPE = 512, 64
 
 
-def _case(lens, H, page, dt, seed=0, ns=4, fused=True, jump=None, bad_page=False):
+def _case(lens, H, page, dt, seed=0, ns=4, fused=True, jump=None, bad_page=False, edit=None):
     g = torch.Generator(device=DEV).manual_seed(seed + sum(lens) + H)
     B = len(lens)
     pages = max(1, -(-max(lens) // page))
@@ -28,6 +28,12 @@ def _case(lens, H, page, dt, seed=0, ns=4, fused=True, jump=None, bad_page=False
     scale = (DV + DPE) ** -0.5
     at = torch.arange(pages * page, device=DEV)
     exp = torch.zeros(B, H, DV, dtype=torch.float64, device=DEV)
+    if edit is not None:  # edit(cache rows of the sequence's tokens, queries of the sequence)
+        for b, n in enumerate(lens):
+            row = table[b].long()[at[:n] // page] * page + at[:n] % page
+            own = rows[row]
+            edit(own, q[b])
+            rows[row] = own
     if bad_page:
         table[0, 0] = B * pages + 7
     for b, n in enumerate(lens):
@@ -74,7 +80,7 @@ def test_workspace_sizes(ns, lens):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 def test_score_jumps(dt):
-    """Tiles far above the reference maximum (fp16: beyond 2^15 times it) go through the rescale."""
+    """Tiles far above the running maximum of the ones before them go through the rescale."""
     lens = [1000, 64, 300]
     for jump in (0, 50, 96):
         out, exp = _case(lens, 128, 64, dt, jump=jump, ns=2)
@@ -94,3 +100,46 @@ def test_large_batches(B, H):
     lens[B // 2] = 1500
     out, exp = _case(lens, H, 16, torch.bfloat16, ns=1)
     _check(out, exp, lens, torch.bfloat16)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mask", ["-inf", "lowest"])
+@pytest.mark.parametrize("lens", [[20000, 100, 3000], [400] * 150])
+def test_masked_prefix(lens, mask, dt):
+    """Tokens masked through a rope dimension: the first tiles of a sequence score -inf for every head, or the
+    type's lowest value times q (-inf in bf16) for every head or one. The others score about 0, or 150
+    below it, or one of them far above the rest. Pieces of several tiles, cut sequences and whole ones."""
+    value = float("-inf") if mask == "-inf" else torch.finfo(dt).min
+    scale = (DV + DPE) ** -0.5
+    for masked in (40, 320):
+        for heads in (slice(None), slice(5, 6)) if mask == "lowest" else (slice(None),):
+            for level, jump in ((0, 0), (-150, 0), (0, 24)):
+                def edit(own, q):
+                    n = own.shape[0]
+                    if n <= masked:
+                        return
+                    own[:, DV] = 0
+                    own[:masked, DV] = value
+                    q[:, DV] = 0
+                    q[heads, DV] = 16
+                    own[:, DV + 1] = level
+                    own[n - 3, DV + 1] = level + jump
+                    q[:, DV + 1] = 1 / scale
+                out, exp = _case(lens, 128, 64, dt, edit=edit)
+                _check(out, exp, lens, dt)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("at", [0, 33, 100, 15000])
+def test_largest_weight_is_exact(at, dt):
+    """A token 2^34 above the rest wherever it stands in its piece: its weight is 1 and the output is its row, to
+    the others' 2^-20."""
+    lens = [20000] * 2
+
+    def edit(own, q):
+        own[:, DV] = 0
+        own[at, DV] = 24  # e^24 ahead of scores of about randn
+        q[:, DV] = (DV + DPE) ** 0.5
+    out, exp = _case(lens, 128, 64, dt, edit=edit)
+    err = float((out.double() - exp).norm() / exp.norm())
+    assert err < 2.0 ** -14, err

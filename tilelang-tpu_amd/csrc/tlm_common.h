@@ -105,6 +105,12 @@ TLM_DEV float xhalf_max(float x) {
                                                   false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
+// the same over lanes l and l ^ 16
+TLM_DEV float xrow_max(float x) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 TLM_DEV float xhalf_sum(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
                                                   false);

@@ -26,9 +26,11 @@
 //     through LDS, and the wave multiplies V^T rows 128 (2 th + dh) .. + 127 of all 32 tokens. The earlier
 //     kernel split the 576 dims four ways, exchanged 160 KB of partial scores per 32 tokens and repeated
 //     the softmax in four waves.
-//   * Softmax against a reference maximum that the waves share: set by a piece's first tile, raised
-//     (O and l rescaled) only when some P of a later tile leaves the 16-bit range's safe part, which a
-//     flag in LDS tells all waves. The common factor cancels in O / l.
+//   * Softmax against the running maximum of each head, so that the largest weight is exactly 1 in 16 bits
+//     and a piece may start with tiles that score -inf: the two token halves' maxima meet in LDS, and O is
+//     rescaled where a head's maximum rose. Against a reference that only the first tile set (kept until some P left
+//     the 16-bit range) that is one barrier more per tile: 16 x 4,000 .. 8,000 tokens 66.4 -> 72.4 us, 8 x
+//     500 .. 4,000 31.5 -> 32.3; its error was larger (2.0e-3 of fp64 against 1.9e-3 here, bf16).
 //   * Tiles stream through a four-stage LDS ring by LDS-DMA (latent rows one 1 KB instruction per token, rope
 //     rows 8 tokens per instruction). The cache rows of 512 tokens at a time are looked up half a block
 //     ahead into an LDS table. 16-byte chunk c of token r sits at c ^ f(r), f(r) = 2 (r % 8) + r / 8 % 2:
@@ -50,8 +52,8 @@ constexpr int MH_LAT = MH_BN * MH_DV * 2;       // bytes of a tile's latent rows
 constexpr int MH_STAGE = MH_LAT + MH_BN * MH_DPE * 2;
 constexpr int MH_NST = 4;
 // Per wave 1 KB: the partner's half scores ([64 lanes] f32x4) and, once the wave has read them, its P^T
-// block ([4 lane groups][16 heads][4 tokens] 16-bit), its 16 maxima / row sums and its flag.
-constexpr int MH_P = MH_NST * MH_STAGE, MH_BOX = 1024, MH_BOX_X = 512, MH_BOX_FLAG = 576;
+// block ([4 lane groups][16 heads][4 tokens] 16-bit) and its 16 maxima / row sums.
+constexpr int MH_P = MH_NST * MH_STAGE, MH_BOX = 1024, MH_BOX_X = 512;
 constexpr int MH_TBL = 512;                     // tokens of a look-up block; two blocks
 constexpr int MH_TBL_TILES = MH_TBL / MH_BN;
 constexpr int MH_ROWS = MH_P + 8 * MH_BOX;
@@ -281,7 +283,6 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
     return box_hg + (uint32_t)((2 * t2 + hh) * MH_BOX + MH_BOX_X + jl * 4);
   };
   const uint32_t row_tbl = s0 + MH_ROWS;
-  constexpr float P_LIMIT = BF16 ? 18446744073709551616.0f : 32768.0f;
   const bool rope_wave = wave < 4;
 
   for (int b = start.seq; b < a.B && seq_before < hi; ++b) {
@@ -429,48 +430,43 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
       const int tok = (t0 + t) * MH_BN + 16 * th + 4 * g;
 #pragma unroll
       for (int i = 0; i < 4; ++i) s[i] = tok + i < L ? s[i] * a.c : -INFINITY;
-      // raise the reference to the tile's maximum over both token halves (uniform over the workgroup)
-      auto raise = [&]() __attribute__((always_inline)) {
+      // the running maximum, over both token halves
+      {
         float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = xhalf_max(xrow_max(mx));
         if (g == 0) ds_put32(x_addr(th, dh), __float_as_uint(mx));
-        mh_barrier();
+      }
+      mh_barrier();
+      uint32_t mt[2][2];  // the tile's maxima: [head tile][token half]
+      asm volatile(
+          "ds_read_b32 %0, %4\n\tds_read_b32 %1, %4 offset:%5\n\tds_read_b32 %2, %4 offset:%6\n\t"
+          "ds_read_b32 %3, %4 offset:%7\n\ts_waitcnt lgkmcnt(0)"
+          : "=&v"(mt[0][0]), "=&v"(mt[1][0]), "=&v"(mt[0][1]), "=&v"(mt[1][1])
+          : "v"(x_addr(0, 0)), "i"(MH_BOX), "i"(2 * MH_BOX), "i"(3 * MH_BOX)
+          : "memory");
+      float al[2];
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
-          float y = m[hh];
-#pragma unroll
-          for (int t2 = 0; t2 < 2; ++t2) y = fmaxf(y, __uint_as_float(ds_get32(x_addr(t2, hh))));
-          const float al = y == -INFINITY ? 1.f : fast_exp2(m[hh] - y);
-          m[hh] = y;
-          if (hh == dh) l *= al;
-#pragma unroll
-          for (int dt = 0; dt < 8; ++dt) oacc[dt][hh] *= al;
-        }
-      };
-      float ps;
-      auto weights = [&]() __attribute__((always_inline)) {
+      for (int hh = 0; hh < 2; ++hh) {
+        const float y = fmaxf(m[hh], fmaxf(__uint_as_float(mt[hh][0]), __uint_as_float(mt[hh][1])));
+        al[hh] = y == -INFINITY ? 1.f : fast_exp2(m[hh] - y);
+        m[hh] = y;
+      }
+      {
         const float mo = dh ? m[1] : m[0];
         const float mm = mo == -INFINITY ? 0.f : mo;
         f32x4 p;
 #pragma unroll
         for (int i = 0; i < 4; ++i) p[i] = fast_exp2(s[i] - mm);
-        ps = (p[0] + p[1]) + (p[2] + p[3]);
+        l = l * (dh ? al[1] : al[0]) + ((p[0] + p[1]) + (p[2] + p[3]));
         ds_put64(box + p_off, u32x2{HH::pack(p[0], p[1]), HH::pack(p[2], p[3])});
-      };
-      if (t == 0) raise();
-      weights();
-      const bool over = __builtin_amdgcn_ballot_w64(!(ps <= P_LIMIT)) != 0;
-      if (lane == 0) ds_put32(box + MH_BOX_FLAG, over);
-      mh_barrier();  // every wave's P^T and flag are in LDS
-      if (__builtin_amdgcn_ballot_w64(
-              ds_get32(s0 + MH_P + MH_BOX_FLAG + (uint32_t)(lane & 7) * MH_BOX) != 0)) {  // rare
-        mh_barrier();
-        raise();
-        weights();
-        mh_barrier();
       }
-      l += ps;
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh)
+        if (__builtin_amdgcn_ballot_w64(!(al[hh] == 1.f))) {  // rarely after a piece's first tiles
+#pragma unroll
+          for (int dt = 0; dt < 8; ++dt) oacc[dt][hh] *= al[hh];
+        }
+      mh_barrier();  // every wave's P^T is in LDS
 
       // ---- O^T += V^T P^T: dims 128 w .. of the wave's 32 heads over the tile's 32 tokens
       u32x2 pb[2][2];  // [head tile][token half]
