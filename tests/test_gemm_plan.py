@@ -1,0 +1,41 @@
+"""Which kernel, tile and split a GEMM call takes (tlm_gemm_plan: host only, no GPU needed)."""
+import ctypes
+
+import pytest
+
+from tilelang.jit.adapter.mi355x import lib
+
+PER_THREAD = 2  # hipStreamPerThread
+
+
+def plan(M, N, K, dt=lib.F16, trans_b=True, dual=False, stream=None, captured=False):
+    out = [ctypes.c_int() for _ in range(3)]
+    lib.call("tlm_gemm_plan", M, N, K, dt, int(trans_b), int(dual), stream, int(captured),
+             *(ctypes.byref(v) for v in out))
+    return tuple(v.value for v in out)
+
+
+SPLIT_CALLS = [dict(M=16, N=14336, K=4096, trans_b=False), dict(M=16, N=4096, K=14336, trans_b=False),
+               dict(M=16, N=4096, K=4096, trans_b=False), dict(M=16, N=4096, K=14336),
+               dict(M=64, N=1024, K=4096, dt=lib.BF16), dict(M=500, N=4096, K=4096, trans_b=False),
+               dict(M=16, N=4096, K=4096, dt=lib.F8E4M3), dict(M=64, N=2048, K=7168, dual=True)]
+
+
+@pytest.mark.parametrize("call", SPLIT_CALLS)
+def test_per_thread_stream_never_splits(call):
+    """hipStreamPerThread is one handle for a stream of every thread: a workspace slot kept by the handle would be
+    shared by calls that overlap."""
+    assert plan(**call)[2] > 1
+    assert plan(**call, stream=0x1000)[2] > 1
+    assert plan(**call, stream=PER_THREAD)[2] == 1
+    assert plan(**call, stream=PER_THREAD, captured=True)[2] == 1
+
+
+def test_plan_rejects_bad_arguments():
+    L = lib.load()
+    v = ctypes.byref(ctypes.c_int())
+    assert L.tlm_gemm_plan(1, 8, 8, lib.F16, 0, 0, None, 0, None, v, v) == -1
+    assert L.tlm_gemm_plan(0, 8, 8, lib.F16, 0, 0, None, 0, v, v, v) == -1
+    assert L.tlm_gemm_plan(1, 8, 8, lib.F32, 0, 0, None, 0, v, v, v) == -2
+    assert L.tlm_gemm_plan(1, 8, 8, lib.F16, 0, 1, None, 0, v, v, v) == -2
+    assert plan(4, 64, 60) == (0, 0, 1)

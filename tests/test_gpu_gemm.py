@@ -138,6 +138,36 @@ def test_gemm_skinny_concurrent_streams():
         torch_assert_close(c.cpu(), ref.matmul_ref(x, y), atol=1e-2, rtol=1e-2)
 
 
+def test_gemm_per_thread_stream():
+    """Calls of several host threads on hipStreamPerThread, one handle for different streams, share no workspace: each
+    repeats the bits of the unsplit call."""
+    import threading
+
+    from tilelang.jit.adapter.mi355x import lib
+    g = torch.Generator(device=DEV).manual_seed(24)
+    ins = [(torch.randn(16, 4096, generator=g, device=DEV).half(),
+            torch.randn(4096, n, generator=g, device=DEV).half()) for n in (4096, 6144, 4096)]
+    outs = [[torch.empty(16, b.shape[1], device=DEV) for _ in range(20)] for _, b in ins]
+    torch.cuda.synchronize()
+
+    def work(i):
+        a, b = ins[i]
+        for c in outs[i]:
+            lib.call("tlm_gemm", a.data_ptr(), b.data_ptr(), c.data_ptr(), 16, b.shape[1], 4096,
+                     lib.F16, lib.F32, 0, 2)  # 2: hipStreamPerThread
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(ins))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for (a, b), cs in zip(ins, outs):
+        exp = a.double() @ b.double()
+        assert float((cs[0].double() - exp).norm() / exp.norm()) < 4 * 64 * 2.0 ** -24
+        assert all(torch.equal(c, cs[0]) for c in cs[1:])
+
+
 def test_gemm_skinny_split_graph_replays():
     """A skinny GEMM captured in a HIP graph (no memset node: the split kernel's arrival counters
     are reset by the kernel) gives, on every replay, the bits of the same call run eagerly on

@@ -700,26 +700,42 @@ int ss_nsplit(int N, int K) {
   return ns;
 }
 
+// What a 16-bit call on 16-byte aligned operands runs: gemm_skinny_split with `skinny` splits, else the tile
+// t (tile -1: gemm_256x256).
+struct Plan16 {
+  int skinny = 0;
+  gt::Plan t{-1, 1};
+  int splits() const { return skinny > 0 ? skinny : t.ns; }
+};
+// One decode step on a large row-major B: the split skinny kernel streams 256-byte rows with A
+// kept in LDS (16 rows: 4096 x 14336 23.5 us against 25.5 on the best tile, 14336 x 4096 24.4
+// against 24.9). Below 32 MB the 32-row tile's shorter start and end win (4096^2 11.6 against
+// 11.7, 2048^2 8.6 against 6.7, 512 x 4096 8.4 against 6.7).
+Plan16 plan16(bool trans_b, int M, int N, int K, bool split) {
+  Plan16 p;
+  if (M <= 16 && !trans_b && (int64_t)N * K * 2 >= (32 << 20) &&
+      (int64_t)(K + 2 * SS_BK) * N * 2 < 0x7ffffff0)
+    p.skinny = ss_nsplit(N, K);
+  if (p.skinny > 1 && !split) p.skinny = 0;
+  if (p.skinny == 0) p.t = gt::plan_tiles(false, trans_b, M, N, K, split);
+  return p;
+}
+
 template <bool BF16, bool TRANS_B, int OUT>
 int launch(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t s) {
   const bool vec = tlm_aligned(A, 16) && tlm_aligned(B, 16) && K % 8 == 0 &&
                    (TRANS_B || N % 8 == 0);
-  // One decode step on a large row-major B: the split skinny kernel streams 256-byte rows with A
-  // kept in LDS (16 rows: 4096 x 14336 23.5 us against 25.5 on the best tile, 14336 x 4096 24.4
-  // against 24.9). Below 32 MB the 32-row tile's shorter start and end win (4096^2 11.6 against
-  // 11.7, 2048^2 8.6 against 6.7, 512 x 4096 8.4 against 6.7).
-  int ns = 0;
+  Plan16 p = vec ? plan16(TRANS_B, M, N, K, true) : Plan16{};
   float* part = nullptr;
   unsigned* arrivals = nullptr;
-  if (vec && M <= 16 && !TRANS_B && (int64_t)N * K * 2 >= (32 << 20) &&
-      (int64_t)(K + 2 * SS_BK) * N * 2 < 0x7ffffff0)
-    ns = ss_nsplit(N, K);
-  if (ns > 1 && !tlm_split_slot(s, &part, &arrivals)) ns = 0;
-  if (ns > 0) {
+  if (p.splits() > 1 && !gt::split_workspace(s, M <= 16, &part, &arrivals))
+    p = plan16(TRANS_B, M, N, K, false);
+  if (p.skinny > 0) {
     const int nstrips = (N + SS_NT - 1) / SS_NT;
-    gemm_skinny_split<BF16, OUT><<<(unsigned)(nstrips * ns), 64 * SS_WAVES, 0, s>>>(
-        (const uint16_t*)A, (const uint16_t*)B, C, M, N, K, ns, part, arrivals);
-  } else if (vec && gt::run_tiles<BF16 ? gt::EL_BF16 : gt::EL_F16, TRANS_B, OUT>(A, B, C, M, N, K, s)) {
+    gemm_skinny_split<BF16, OUT><<<(unsigned)(nstrips * p.skinny), 64 * SS_WAVES, 0, s>>>(
+        (const uint16_t*)A, (const uint16_t*)B, C, M, N, K, p.skinny, part, arrivals);
+  } else if (gt::run_tiles<BF16 ? gt::EL_BF16 : gt::EL_F16, TRANS_B, OUT>(p.t, A, B, C, M, N, K, part,
+                                                                         arrivals, s)) {
     // between one decode step and a whole prompt batch
   } else if (vec && (int64_t)BM * K * 2 < 0x7ffffff0 &&
              (TRANS_B ? (int64_t)BN * K * 2 : (int64_t)BK * N * 2) < 0x7ffffff0) {
@@ -787,9 +803,42 @@ extern "C" int tlm_gemm(const void* A, const void* B, void* C, int64_t M, int64_
                  : by_out<false, false>(A, B, C, m, n, k, out_dtype, s);
 }
 
+extern "C" int tlm_gemm_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int trans_b, int dual,
+                             void* stream, int captured, int* rows, int* cols, int* splits) {
+  const bool fp8 = in_dtype == TLM_F8E4M3 || in_dtype == TLM_F8E5M2;
+  if (!rows || !cols || !splits) {
+    tlm_set_error("tlm_gemm_plan: null pointer argument");
+    return TLM_EINVAL;
+  }
+  if (M <= 0 || N <= 0 || K < 0 || M > INT32_MAX || N > INT32_MAX / 2 || K > INT32_MAX) {
+    tlm_set_error("tlm_gemm_plan: bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N,
+                  (long long)K);
+    return TLM_EINVAL;
+  }
+  if ((!fp8 && in_dtype != TLM_F16 && in_dtype != TLM_BF16) || (dual && (fp8 || !trans_b))) {
+    tlm_set_error("tlm_gemm_plan: in_dtype %d unsupported", in_dtype);
+    return TLM_EUNSUPPORTED;
+  }
+  *rows = *cols = 0;
+  *splits = 1;
+  if (fp8 ? !trans_b || K % 16 : K % 8 || (!trans_b && N % 8)) return TLM_OK;
+  const bool split = gt::may_split((hipStream_t)stream, captured != 0, !fp8 && !dual && M <= 16);
+  Plan16 p;
+  if (dual)
+    p.t = gt::dual_plan(M, N, K, split);
+  else if (fp8)
+    p.t = gt::plan_tiles(true, true, M, N, K, split);
+  else
+    p = plan16(trans_b != 0, (int)M, (int)N, (int)K, split);
+  *splits = p.splits();
+  *rows = p.skinny > 0 ? 16 : p.t.tile < 0 ? 256 : gt::SHAPES[p.t.tile].bm;
+  *cols = p.skinny > 0 ? SS_NT : p.t.tile < 0 ? 256 : gt::SHAPES[p.t.tile].bn;
+  return TLM_OK;
+}
+
 extern "C" size_t tlm_gemm_swiglu_tmp_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K < 0 || M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return 0;
-  return gt::dual_plan(M, N, K).tile < 0 ? (size_t)M * N * 2 : 0;
+  return gt::dual_plan(M, N, K, true).tile < 0 ? (size_t)M * N * 2 : 0;
 }
 
 extern "C" int tlm_gemm_swiglu(const void* A, const void* B_gate, const void* B_up, void* H,
@@ -816,7 +865,7 @@ extern "C" int tlm_gemm_swiglu(const void* A, const void* B_gate, const void* B_
   if (M == 0 || N == 0) return TLM_OK;
   hipStream_t s = (hipStream_t)stream;
   if (tlm_aligned(A, 16) && tlm_aligned(B_gate, 16) && tlm_aligned(B_up, 16)) {
-    const gt::Plan p = gt::dual_plan(M, N, K);
+    const gt::Plan p = gt::dual_plan(M, N, K, true);
     if (p.tile >= 0) {
       if (dtype == TLM_BF16)
         gt::run_swiglu<gt::EL_BF16, TLM_BF16>(p, A, B_gate, B_up, H, (int)M, (int)N, (int)K, s);

@@ -365,7 +365,13 @@ int launch(const void* A, const void* B, void* C, int M, int N, int K, bool tran
   // 32-bit LDS-DMA byte offsets r * K + 16 c within a 256-row panel stay below the
   // descriptor's num_records (2^31 - 16): K < 2^23
   const bool tiled = vec && M > 16 && K < (1 << 23);
-  if (vec && gt::run_tiles<FMT == 0 ? gt::EL_E4M3 : gt::EL_E5M2, true, OUT>(A, B, C, M, N, K, s)) {
+  gt::Plan p = vec ? gt::plan_tiles(true, true, M, N, K, true) : gt::Plan{-1, 1};
+  float* part = nullptr;
+  unsigned* arrivals = nullptr;
+  if (p.ns > 1 && !gt::split_workspace(s, false, &part, &arrivals))
+    p = gt::plan_tiles(true, true, M, N, K, false);
+  if (gt::run_tiles<FMT == 0 ? gt::EL_E4M3 : gt::EL_E5M2, true, OUT>(p, A, B, C, M, N, K, part, arrivals,
+                                                                    s)) {
     // tlm_gemm_tile.h: the shapes whose 256x256 tiles would not fill the chip
   } else if (tiled) {
     const int64_t tiles = (int64_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN);

@@ -678,32 +678,34 @@ void launch_tile(const void* A, const void* B, void* C, int M, int N, int K, int
                                                       K, ns, part, arrivals, B2);
 }
 
-// Whether a split may run on stream `s` (a 16-bit call with M <= 16 also inside a capture), and its
-// workspace.
-inline bool split_workspace(hipStream_t s, bool in_capture, float** part, unsigned** arrivals) {
-  if (s == hipStreamPerThread) return false;  // one handle for a stream of every thread
-  if (!in_capture) {
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
-  }
-  return tlm_split_slot(s, part, arrivals);
+// Whether a call on stream `s` may split K. hipStreamPerThread is one handle for a stream of every thread, so
+// it can own no workspace. Inside a capture only calls that may keep the captured stream's workspace
+// (`graph_ok`) split, so that other graphs captured on one stream may be replayed side by side.
+inline bool may_split(hipStream_t s, bool captured, bool graph_ok) {
+  return s != hipStreamPerThread && (graph_ok || !captured);
+}
+inline bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+inline bool split_workspace(hipStream_t s, bool graph_ok, float** part, unsigned** arrivals) {
+  return may_split(s, s != hipStreamPerThread && !graph_ok && capturing(s), graph_ok) &&
+         tlm_split_slot(s, part, arrivals);
 }
 
-// Runs the plan's tile; false when the plan is the 256 x 256 kernel (or the shape does not fit the tiles'
-// 32-bit offsets). The caller checked the alignment. 16-bit calls with M <= 16 may keep a captured
-// stream's workspace, as its callers are told; others never split inside a capture, so graphs captured
-// on one stream may be replayed side by side.
-template <int EL, bool TB, int OUT>
-bool run_tiles(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t s) {
-  constexpr bool FP8 = EL >= EL_E4M3;
+// The tile and split of a call on 16-byte aligned operands; tile -1: the 256 x 256 kernel (also where the shape
+// does not fit the tiles' 32-bit offsets).
+inline Plan plan_tiles(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, bool split) {
   constexpr int64_t LIM = 0x7ffffff0;
-  if (256 * (int64_t)K * (FP8 ? 1 : 2) >= LIM || (!TB && 128 * (int64_t)N * 2 >= LIM) || K <= 0)
-    return false;
-  Plan p = choose(FP8, TB, M, N, K, 16);
-  float* part = nullptr;
-  unsigned* arrivals = nullptr;
-  if (p.ns > 1 && !split_workspace(s, M <= 16 && !FP8, &part, &arrivals))
-    p = choose(FP8, TB, M, N, K, 1);
+  if (256 * K * (fp8 ? 1 : 2) >= LIM || (!trans_b && 128 * N * 2 >= LIM) || K <= 0) return Plan{-1, 1};
+  return choose(fp8, trans_b, M, N, K, split ? 16 : 1);
+}
+
+// Runs the plan's tile; false for tile -1.
+template <int EL, bool TB, int OUT>
+bool run_tiles(Plan p, const void* A, const void* B, void* C, int M, int N, int K, float* part,
+               unsigned* arrivals, hipStream_t s) {
+  constexpr bool FP8 = EL >= EL_E4M3;
   switch (p.tile) {
     case T32:
       // 16 rows or fewer of fp8 are multiplied as fp16, which costs nothing beside B's stream and
@@ -731,17 +733,19 @@ bool run_tiles(const void* A, const void* B, void* C, int M, int N, int K, hipSt
 // ---- up * silu(gate) of two products with one A: gate = A B^T, up = A B2^T, both [M, N]. The MLP of
 // 64 tokens (7168 x 2048) spent its time in launches and their gaps: two products, SwiGLU (4.6 us for
 // 0.8 MB) and the down product took 46.5 us; with the first three in one kernel 27.3.
-inline Plan dual_plan(int64_t M, int64_t N, int64_t K) {
+// Without a split a call that may not split still takes a tile, so that tlm_gemm_swiglu_tmp_bytes holds for
+// every stream.
+inline Plan dual_plan(int64_t M, int64_t N, int64_t K, bool split) {
   if (256 * K * 2 >= 0x7ffffff0 || K <= 0 || K % 8) return Plan{-1, 1};
-  return choose(false, true, M, 2 * N, K, 16, true);
+  const Plan p = choose(false, true, M, 2 * N, K, 16, true);
+  return p.tile < 0 || p.ns == 1 || split ? p : choose(false, true, M, 2 * N, K, 1, true, true);
 }
 template <int EL, int OUT>
 void run_swiglu(Plan p, const void* A, const void* B, const void* B2, void* C, int M, int N, int K,
                 hipStream_t s) {
   float* part = nullptr;
   unsigned* arrivals = nullptr;
-  if (p.ns > 1 && !split_workspace(s, false, &part, &arrivals))
-    p = choose(false, true, M, 2 * (int64_t)N, K, 1, true, true);
+  if (p.ns > 1 && !split_workspace(s, false, &part, &arrivals)) p = dual_plan(M, N, K, false);
   const uint8_t* const b2 = (const uint8_t*)B2;
   switch (p.tile) {
     case T32W:

@@ -35,6 +35,8 @@ _SIGNATURES = {
     "tlm_gemm": ([c_void_p] * 3 + [c_int64] * 3 + [c_int] * 3 + [c_void_p], c_int),
     "tlm_gemm_swiglu_tmp_bytes": ([c_int64] * 3, c_size_t),
     "tlm_gemm_swiglu": ([c_void_p] * 5 + [c_int64] * 3 + [c_int, c_void_p], c_int),
+    "tlm_gemm_plan": ([c_int64] * 3 + [c_int] * 3 + [c_void_p, c_int] +
+                      [ctypes.POINTER(c_int)] * 3, c_int),
     "tlm_gemm_fp8": ([c_void_p] * 3 + [c_int64] * 3 + [c_int] * 3 + [c_void_p], c_int),
     "tlm_flash_attn_fwd": ([c_void_p] * 4 + [c_int64] * 4 + [c_int, c_float, c_int, c_void_p],
                            c_int),
