@@ -39,3 +39,26 @@ def test_plan_rejects_bad_arguments():
     assert L.tlm_gemm_plan(1, 8, 8, lib.F32, 0, 0, None, 0, v, v, v) == -2
     assert L.tlm_gemm_plan(1, 8, 8, lib.F16, 0, 1, None, 0, v, v, v) == -2
     assert plan(4, 64, 60) == (0, 0, 1)
+
+
+def test_captured_calls_that_may_keep_the_streams_workspace():
+    """Two graphs captured on one stream may be replayed side by side unless they hold a call that keeps the
+    stream's workspace: 16 rows or fewer of 16 bits, B^T of up to 8,192 columns (128 strips of 64) and row-major
+    B of up to 16,384 (128 strips of 128) or more than 2,048 of k. No other call splits inside a capture."""
+    for M in (1, 16):
+        for K in (64, 256, 480, 512, 2048, 2056, 4096, 7168, 14336, 28672):
+            for N in (64, 1000, 4096, 8192, 8200, 9000, 10496, 12288, 16384, 16392, 20480, 28672):
+                for dt in (lib.F16, lib.BF16):
+                    if N > 8192 or K <= 480:
+                        assert plan(M, N, K, dt, captured=True)[2] == 1, (M, N, K)
+                    if N > 16384 and K <= 2048:
+                        assert plan(M, N, K, dt, trans_b=False, captured=True)[2] == 1, (M, N, K)
+                assert plan(M, N, K, lib.F8E4M3, captured=True)[2] == 1
+                assert plan(M, N, K, lib.BF16, dual=True, captured=True)[2] == 1
+                for rows in (17, 64, 500):
+                    for tb in (False, True):
+                        assert plan(rows, N, K, trans_b=tb, captured=True)[2] == 1
+    # those that kept it still split
+    assert plan(16, 4096, 14336, captured=True)[2] > 1
+    assert plan(16, 14336, 4096, trans_b=False, captured=True)[2] > 1
+    assert plan(16, 4096, 4096, trans_b=False, captured=True)[2] > 1

@@ -721,6 +721,15 @@ Plan16 plan16(bool trans_b, int M, int N, int K, bool split) {
   return p;
 }
 
+// Calls whose split may keep the workspace of a captured stream: those of one decode step, whose callers are told
+// to replay such graphs one after the other. B^T wider than 128 strips of 64 columns and row-major B that one
+// workgroup per strip of 128 columns covers are not among them, nor is anything above 16 rows.
+bool graph_split(bool trans_b, int M, int N, int K) {
+  if (M > 16) return false;
+  if (trans_b) return N <= 128 * 64 && K > 480;
+  return (int64_t)(K + 2 * SS_BK) * N * 2 < 0x7ffffff0 && ss_nsplit(N, K) > 1;
+}
+
 template <bool BF16, bool TRANS_B, int OUT>
 int launch(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t s) {
   const bool vec = tlm_aligned(A, 16) && tlm_aligned(B, 16) && K % 8 == 0 &&
@@ -728,7 +737,7 @@ int launch(const void* A, const void* B, void* C, int M, int N, int K, hipStream
   Plan16 p = vec ? plan16(TRANS_B, M, N, K, true) : Plan16{};
   float* part = nullptr;
   unsigned* arrivals = nullptr;
-  if (p.splits() > 1 && !gt::split_workspace(s, M <= 16, &part, &arrivals))
+  if (p.splits() > 1 && !gt::split_workspace(s, graph_split(TRANS_B, M, N, K), &part, &arrivals))
     p = plan16(TRANS_B, M, N, K, false);
   if (p.skinny > 0) {
     const int nstrips = (N + SS_NT - 1) / SS_NT;
@@ -822,7 +831,9 @@ extern "C" int tlm_gemm_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int 
   *rows = *cols = 0;
   *splits = 1;
   if (fp8 ? !trans_b || K % 16 : K % 8 || (!trans_b && N % 8)) return TLM_OK;
-  const bool split = gt::may_split((hipStream_t)stream, captured != 0, !fp8 && !dual && M <= 16);
+  const bool split =
+      gt::may_split((hipStream_t)stream, captured != 0,
+                    !fp8 && !dual && graph_split(trans_b != 0, (int)M, (int)N, (int)K));
   Plan16 p;
   if (dual)
     p.t = gt::dual_plan(M, N, K, split);
