@@ -108,12 +108,13 @@ int tlm_rope(const void* q, const void* k, const void* cos_t, const void* sin_t,
  * (tpu_demo/matmul/tpu_test_matmul_fp32.py:9-31) copies its fp32 A/B tiles to fp16 before
  * ppl_gemm: tlm_cast to F16, then this with out_dtype F32.
  * Calls whose tiles are fewer than the CUs split K over several workgroups, whose partial tiles
- * meet in a library-owned device workspace (64 MB per GPU, 4 slots): each stream owns one slot,
- * so calls on one stream are ordered and calls that overlap use different slots; further streams
+ * meet in a library-owned device workspace (96 MB per GPU: 4 slots for calls with M <= 16, 4 for
+ * larger and fp8 calls): each stream owns a slot of each kind that it uses, so calls on one
+ * stream are ordered and calls that overlap use different slots; further streams
  * (and hipStreamPerThread) run unsplit. Inside a stream capture only M <= 16 may split (B^T: up to
  * 8,192 columns; row-major B: up to 16,384 columns or above 2,048 of K): such a HIP graph keeps
  * the slot of the stream it was captured on, so its replays must not overlap each other or other
- * work of that stream; all other calls are captured unsplit. Slots are keyed by the
+ * such calls of that stream; all other calls are captured unsplit. Slots are keyed by the
  * stream handle: a stream created after another is destroyed can get the same handle and inherits
  * its slot, so a stream is destroyed only once its calls have finished. The result does not depend
  * on the split's timing: a stream's calls are bitwise reproducible (a call that runs unsplit sums

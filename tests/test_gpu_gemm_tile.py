@@ -6,9 +6,13 @@ Tolerance: fp32 sums of K products with |partial sums| <= s err by at most K ulp
 relative 2-norm error stays below 4 sqrt(K) 2^-24, plus half an ulp of the output type (2^-9 bf16,
 2^-12 fp16). fp8 above 16 rows: the fp8 matrix instruction drops low bits of its sums (measured 1.3e-5).
 """
+import subprocess
+import sys
+
 import pytest
 import torch
 
+from conftest import PKG
 from tilelang.jit.adapter.mi355x import ops
 
 pytestmark = pytest.mark.gpu
@@ -130,3 +134,35 @@ def test_gemm_swiglu(M, N, K, dt):
         ops.gemm_swiglu(a, bg, bu, h)
         gate, up = a.double() @ bg.double().T, a.double() @ bu.double().T
         assert _rel(h, up * gate * torch.sigmoid(gate)) < 3 * ULP[dt]
+
+
+DECODE_SLOTS = """
+import torch
+from tilelang.jit.adapter.mi355x import ops
+g = torch.Generator(device="cuda").manual_seed(5)
+x = torch.randn(64, 4096, generator=g, device="cuda").half()
+w = torch.randn(2048, 4096, generator=g, device="cuda").half()
+streams = [torch.cuda.Stream() for _ in range(4)]
+torch.cuda.synchronize()
+for st in streams:  # split calls of 64 rows own a workspace each
+    with torch.cuda.stream(st):
+        ops.gemm(x, w, torch.empty(64, 2048, device="cuda"), trans_b=True)
+torch.cuda.synchronize()
+res = []
+for i in range(6):
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        res.append(ops.gemm(x[:16], w, torch.empty(16, 2048, device="cuda"), trans_b=True))
+    streams.append(st)  # kept: a handle is not used again
+torch.cuda.synchronize()
+print("EQUAL", [bool(torch.equal(r, res[0])) for r in res])
+"""
+
+
+def test_decode_calls_keep_their_workspaces_beside_larger_calls():
+    """Streams that run split calls of more than 16 rows take none of the four slots of decode steps: four further
+    streams still split them (the bits of one call), the streams after those run unsplit (others)."""
+    r = subprocess.run([sys.executable, "-c", DECODE_SLOTS], capture_output=True, text=True, timeout=100,
+                       cwd=PKG)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert "EQUAL [True, True, True, True, False, False]" in r.stdout, r.stdout

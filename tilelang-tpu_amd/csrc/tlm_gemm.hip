@@ -432,7 +432,7 @@ constexpr int SS_NT = 128;
 constexpr int SS_BK = 16;
 constexpr int SS_AMAX_K = 2048;  // k range of one workgroup: its A is 64 KB of LDS
 constexpr int SS_MAX_SPLIT = 16;
-constexpr int SS_SLOTS = 4;      // workspace slots, one per stream
+constexpr int SS_SLOTS = 4;      // workspace slots of each kind, one per stream
 constexpr int SS_MAX_WG = 512;   // workgroups of one call that publish a partial tile
 constexpr int SS_PART = 16 * SS_NT;
 
@@ -630,24 +630,29 @@ __global__ __launch_bounds__(256) void gemm_generic(const uint16_t* __restrict__
 }  // namespace
 
 // Workspace of the split kernels, one instance per GPU (a device that loads this code object
-// holds its own copy until the process ends; 64 MB): SS_SLOTS slots of partial tiles and arrival
-// counters. The counters start at zero and every call leaves them at zero. In host code the names
-// only identify the symbols; the device addresses come from hipGetSymbolAddress.
-static __device__ __align__(256) float ss_partials[SS_SLOTS][TLM_SPLIT_BYTES / 4];
-static __device__ __align__(256) unsigned ss_arrivals[SS_SLOTS][TLM_SPLIT_TILES];
-static_assert(SS_MAX_WG <= TLM_SPLIT_TILES && (size_t)SS_MAX_WG * SS_PART * 4 <= TLM_SPLIT_BYTES,
+// holds its own copy until the process ends; 96 MB): SS_SLOTS slots of partial tiles and arrival
+// counters for the calls of one decode step and as many for the others. The counters start at zero and
+// every call leaves them at zero. In host code the names only identify the symbols; the device
+// addresses come from hipGetSymbolAddress.
+static __device__ __align__(256) float ss_partials[SS_SLOTS][tlm_split_bytes(true) / 4];
+static __device__ __align__(256) float tile_partials[SS_SLOTS][tlm_split_bytes(false) / 4];
+static __device__ __align__(256) unsigned split_arrivals[2][SS_SLOTS][TLM_SPLIT_TILES];
+static_assert(SS_MAX_WG <= TLM_SPLIT_TILES && (size_t)SS_MAX_WG * SS_PART * 4 <= tlm_split_bytes(true),
               "the skinny kernel's tiles fit a slot");
 
 namespace {
 
 constexpr int kSsDevices = 64;
-struct SsDevice {
-  std::once_flag once;
-  hipError_t err = hipSuccess;
+struct SsPool {
   float* part = nullptr;
   unsigned* arrivals = nullptr;
   bool used[SS_SLOTS] = {};
   hipStream_t owner[SS_SLOTS] = {};
+};
+struct SsDevice {
+  std::once_flag once;
+  hipError_t err = hipSuccess;
+  SsPool pool[2];  // the calls of one decode step; the others
 };
 SsDevice g_ss[kSsDevices];
 std::mutex g_ss_mu;
@@ -656,32 +661,35 @@ std::mutex g_ss_mu;
 
 // The workspace slot of stream `s` on the current device: the one it owns, else a free one that
 // it then owns. False when every slot is owned by another stream (or the lookup failed).
-bool tlm_split_slot(hipStream_t s, float** part, unsigned** arrivals) {
+bool tlm_split_slot(bool decode, hipStream_t s, float** part, unsigned** arrivals) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kSsDevices) return false;
   SsDevice& d = g_ss[dev];
   std::call_once(d.once, [&d]() {
-    void* p = nullptr;
-    void* q = nullptr;
-    d.err = hipGetSymbolAddress(&p, HIP_SYMBOL(ss_partials));
-    if (d.err == hipSuccess) d.err = hipGetSymbolAddress(&q, HIP_SYMBOL(ss_arrivals));
-    d.part = (float*)p;
-    d.arrivals = (unsigned*)q;
+    void* p[3] = {};
+    d.err = hipGetSymbolAddress(&p[0], HIP_SYMBOL(ss_partials));
+    if (d.err == hipSuccess) d.err = hipGetSymbolAddress(&p[1], HIP_SYMBOL(tile_partials));
+    if (d.err == hipSuccess) d.err = hipGetSymbolAddress(&p[2], HIP_SYMBOL(split_arrivals));
+    for (int i = 0; i < 2; ++i) {
+      d.pool[i].part = (float*)p[i];
+      d.pool[i].arrivals = (unsigned*)p[2] + (size_t)i * SS_SLOTS * TLM_SPLIT_TILES;
+    }
   });
   if (d.err != hipSuccess) return false;
+  SsPool& q = d.pool[decode ? 0 : 1];
   std::lock_guard<std::mutex> lk(g_ss_mu);
   int slot = -1;
   for (int i = 0; i < SS_SLOTS && slot < 0; ++i)
-    if (d.used[i] && d.owner[i] == s) slot = i;
+    if (q.used[i] && q.owner[i] == s) slot = i;
   for (int i = 0; i < SS_SLOTS && slot < 0; ++i)
-    if (!d.used[i]) {
-      d.used[i] = true;
-      d.owner[i] = s;
+    if (!q.used[i]) {
+      q.used[i] = true;
+      q.owner[i] = s;
       slot = i;
     }
   if (slot < 0) return false;
-  *part = d.part + (size_t)slot * (TLM_SPLIT_BYTES / 4);
-  *arrivals = d.arrivals + (size_t)slot * TLM_SPLIT_TILES;
+  *part = q.part + (size_t)slot * (tlm_split_bytes(decode) / 4);
+  *arrivals = q.arrivals + (size_t)slot * TLM_SPLIT_TILES;
   return true;
 }
 
@@ -737,7 +745,7 @@ int launch(const void* A, const void* B, void* C, int M, int N, int K, hipStream
   Plan16 p = vec ? plan16(TRANS_B, M, N, K, true) : Plan16{};
   float* part = nullptr;
   unsigned* arrivals = nullptr;
-  if (p.splits() > 1 && !gt::split_workspace(s, graph_split(TRANS_B, M, N, K), &part, &arrivals))
+  if (p.splits() > 1 && !gt::split_workspace(M <= 16, s, graph_split(TRANS_B, M, N, K), &part, &arrivals))
     p = plan16(TRANS_B, M, N, K, false);
   if (p.skinny > 0) {
     const int nstrips = (N + SS_NT - 1) / SS_NT;

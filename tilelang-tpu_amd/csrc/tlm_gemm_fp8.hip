@@ -368,7 +368,7 @@ int launch(const void* A, const void* B, void* C, int M, int N, int K, bool tran
   gt::Plan p = vec ? gt::plan_tiles(true, true, M, N, K, true) : gt::Plan{-1, 1};
   float* part = nullptr;
   unsigned* arrivals = nullptr;
-  if (p.ns > 1 && !gt::split_workspace(s, false, &part, &arrivals))
+  if (p.ns > 1 && !gt::split_workspace(false, s, false, &part, &arrivals))
     p = gt::plan_tiles(true, true, M, N, K, false);
   if (gt::run_tiles<FMT == 0 ? gt::EL_E4M3 : gt::EL_E5M2, true, OUT>(p, A, B, C, M, N, K, part, arrivals,
                                                                     s)) {

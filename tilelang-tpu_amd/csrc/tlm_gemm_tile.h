@@ -27,12 +27,14 @@
 
 #include <type_traits>
 
-// Workspace of the split kernels for stream `s` on the current device (tlm_gemm.hip): TLM_SPLIT_BYTES of
+// Workspace of the split kernels for stream `s` on the current device (tlm_gemm.hip): tlm_split_bytes of
 // partial tiles and TLM_SPLIT_TILES zeroed counters that a kernel leaves at zero. False when the
-// stream owns none and none is free.
-constexpr size_t TLM_SPLIT_BYTES = (size_t)16 << 20;
+// stream owns none and none is free. 16-bit calls of one decode step (`decode`: 16 rows or fewer) have
+// slots of their own: streams that run larger calls or fp8 do not take them, and a graph that keeps
+// one can be replayed beside the larger calls of the stream it was captured on.
+constexpr size_t tlm_split_bytes(bool decode) { return (size_t)(decode ? 8 : 16) << 20; }
 constexpr int TLM_SPLIT_TILES = 512;
-bool tlm_split_slot(hipStream_t s, float** part, unsigned** arrivals);
+bool tlm_split_slot(bool decode, hipStream_t s, float** part, unsigned** arrivals);
 
 namespace gt {
 
@@ -227,7 +229,7 @@ constexpr int out_size() {
 // Requires: A, B 16-byte aligned, rows of A (and B^T) and row-major B's rows whole 16-byte chunks,
 // BM K and BN K (B^T) or BK N (row-major) bytes below 2^31 - 16; ns > 1: part and
 // arrivals of tlm_split_slot with grid tiles <= TLM_SPLIT_TILES and grid * BM * BN * 4 <=
-// TLM_SPLIT_BYTES. Grid: ns * ceil(M / BM) * ceil(N / BN) workgroups of THREADS.
+// tlm_split_bytes. Grid: ns * ceil(M / BM) * ceil(N / BN) workgroups of THREADS.
 template <typename CF, int OUT>
 __global__ __launch_bounds__(THREADS, 1) void gemm_tile(const uint8_t* __restrict__ A,
                                                        const uint8_t* __restrict__ B,
@@ -642,6 +644,7 @@ inline Plan choose(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, int 
   };
   const Cost* const cost = fp8 ? C8 : C16;
   const bool only32 = fp8 && M <= 16;  // the one tile with an fp16 product
+  const size_t part_bytes = tlm_split_bytes(!fp8 && !dual && M <= 16);
   Plan best{-1, 1};
   double t_best = only32 || only_tiles ? 1e300 : run(cost[T_COUNT], tiles(256, 256), (kb + 127) / 128);
   if (dual) t_best += 10.0 + (double)M * (double)N * 3e-6 / 6.0;  // two more launches, SwiGLU's bytes
@@ -656,7 +659,7 @@ inline Plan choose(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, int 
     for (int ns = 1; ns <= max_ns; ++ns) {
       const int64_t wg = tl * ns;
       if (ns > 1 && (wg > TLM_SPLIT_TILES || kt < 2 * ns ||
-                     (size_t)wg * s.bm * s.bn * 4 > TLM_SPLIT_BYTES))
+                     (size_t)wg * s.bm * s.bn * 4 > part_bytes))
         break;
       double t_us = run(cost[t], wg, (kt + ns - 1) / ns);
       if (ns > 1)
@@ -688,9 +691,10 @@ inline bool capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
-inline bool split_workspace(hipStream_t s, bool graph_ok, float** part, unsigned** arrivals) {
+inline bool split_workspace(bool decode, hipStream_t s, bool graph_ok, float** part,
+                            unsigned** arrivals) {
   return may_split(s, s != hipStreamPerThread && !graph_ok && capturing(s), graph_ok) &&
-         tlm_split_slot(s, part, arrivals);
+         tlm_split_slot(decode, s, part, arrivals);
 }
 
 // The tile and split of a call on 16-byte aligned operands; tile -1: the 256 x 256 kernel (also where the shape
@@ -745,7 +749,7 @@ void run_swiglu(Plan p, const void* A, const void* B, const void* B2, void* C, i
                 hipStream_t s) {
   float* part = nullptr;
   unsigned* arrivals = nullptr;
-  if (p.ns > 1 && !split_workspace(s, false, &part, &arrivals)) p = dual_plan(M, N, K, false);
+  if (p.ns > 1 && !split_workspace(false, s, false, &part, &arrivals)) p = dual_plan(M, N, K, false);
   const uint8_t* const b2 = (const uint8_t*)B2;
   switch (p.tile) {
     case T32W:
