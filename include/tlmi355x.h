@@ -136,7 +136,8 @@ int tlm_gemm_swiglu(const void* A, const void* B_gate, const void* B_up, void* H
 /* What tlm_gemm, tlm_gemm_fp8 (in_dtype F8E4M3 | F8E5M2) or, with dual != 0, tlm_gemm_swiglu runs for a shape
  * on 16-byte aligned operands: the rows and columns of its tile and the number of workgroups that split
  * K. 16 x 128 is the kernel of one decode step, 256 x 256 the one of whole prompt batches (for
- * tlm_gemm_swiglu the three calls), 0 x 0 one thread per output (K or N not whole 16-byte rows). `captured`:
+ * tlm_gemm_swiglu the three calls), 0 x 0 one thread per output (K or N not whole 16-byte rows, or past
+ * the tiles' launch limits). `captured`:
  * the stream is being captured. A call whose stream finds no workspace slot runs as one that may not
  * split. Host only, no HIP call. */
 int tlm_gemm_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int trans_b, int dual, void* stream,

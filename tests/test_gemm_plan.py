@@ -62,3 +62,15 @@ def test_captured_calls_that_may_keep_the_streams_workspace():
     assert plan(16, 4096, 14336, captured=True)[2] > 1
     assert plan(16, 14336, 4096, trans_b=False, captured=True)[2] > 1
     assert plan(16, 4096, 4096, trans_b=False, captured=True)[2] > 1
+
+
+@pytest.mark.parametrize("M", [1, 17, 32, 64, 100, 300])
+@pytest.mark.parametrize("dt", [lib.F16, lib.F8E4M3])
+def test_no_grid_above_the_launch_limit(M, dt):
+    """A launch counts its threads in 32 bits; very wide calls that 256 x 256 tiles (or one thread per output)
+    cover within it do not take smaller tiles that exceed it."""
+    for N in (1 << 28, 1 << 29, (1 << 29) + 4096, 600_000_000, 1 << 30):
+        for K in (16, 64, 128, 256, 512):
+            rows, cols, ns = plan(M, N, K, dt)
+            if 0 < rows and (rows, cols) != (256, 256):
+                assert -(-M // rows) * -(-N // cols) * ns * 512 < 1 << 32, (N, K, rows, cols)

@@ -827,7 +827,7 @@ extern "C" int tlm_gemm_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int 
     tlm_set_error("tlm_gemm_plan: null pointer argument");
     return TLM_EINVAL;
   }
-  if (M <= 0 || N <= 0 || K < 0 || M > INT32_MAX || N > INT32_MAX / 2 || K > INT32_MAX) {
+  if (M <= 0 || N <= 0 || K < 0 || M > INT32_MAX || N > INT32_MAX / (dual ? 2 : 1) || K > INT32_MAX) {
     tlm_set_error("tlm_gemm_plan: bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N,
                   (long long)K);
     return TLM_EINVAL;
@@ -849,6 +849,7 @@ extern "C" int tlm_gemm_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int 
     p.t = gt::plan_tiles(true, true, M, N, K, split);
   else
     p = plan16(trans_b != 0, (int)M, (int)N, (int)K, split);
+  if (fp8 && p.t.tile < 0 && (M <= 16 || K >= (1 << 23))) return TLM_OK;
   *splits = p.splits();
   *rows = p.skinny > 0 ? 16 : p.t.tile < 0 ? 256 : gt::SHAPES[p.t.tile].bm;
   *cols = p.skinny > 0 ? SS_NT : p.t.tile < 0 ? 256 : gt::SHAPES[p.t.tile].bn;

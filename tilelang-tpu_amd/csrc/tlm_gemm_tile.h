@@ -658,6 +658,7 @@ inline Plan choose(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, int 
     const int64_t tl = tiles(s.bm, s.bn), kt = (kb + s.bkb - 1) / s.bkb;
     for (int ns = 1; ns <= max_ns; ++ns) {
       const int64_t wg = tl * ns;
+      if (wg * THREADS > UINT32_MAX) break;  // a launch counts its threads in 32 bits
       if (ns > 1 && (wg > TLM_SPLIT_TILES || kt < 2 * ns ||
                      (size_t)wg * s.bm * s.bn * 4 > part_bytes))
         break;
