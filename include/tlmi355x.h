@@ -376,6 +376,10 @@ int tlm_mla_decode_ex(const void* q, const void* q_pe, int64_t q_stride, int64_t
 /* Workspace bytes that tlm_mla_decode and tlm_mla_decode_ex need for (B, Hq, dv, num_split). */
 size_t tlm_mla_workspace_bytes(int64_t B, int64_t Hq, int64_t dv, int num_split);
 
+/* Ranges that a decode of B sequences and Hq heads over a 16-bit cache is balanced over with a
+ * workspace of ws_bytes: each is one workgroup per 64 heads. Host only, no HIP call. */
+int64_t tlm_mla_h16_ranges(int64_t B, int64_t Hq, size_t ws_bytes);
+
 /* Bytes of the library-owned scratch of tlm_mla_decode_noalloc (per GPU). */
 #define TLM_MLA_SCRATCH_BYTES ((size_t)128 << 20)
 

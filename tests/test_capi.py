@@ -357,3 +357,19 @@ def test_elementwise_validation():
     assert run([load0, store0], bcast=(I * 1)(9)) == -1  # broadcast kind
     assert run([]) == -1
     assert run([load0] * 65) == -1
+
+
+def test_mla_h16_ranges_fit_the_cus():
+    """A decode workgroup holds a CU's whole LDS: the ranges times the blocks of 64 heads are at most the 256 CUs
+    (the rest would start when the first end), and their partial rows fit the workspace."""
+    L = lib.load()
+    for hq in range(64, 4097, 64):
+        for B in (1, 2, 8, 60, 300, 4096):
+            for ns in (1, 4, 64):
+                ws = L.tlm_mla_workspace_bytes(B, hq, 512, ns)
+                G = L.tlm_mla_h16_ranges(B, hq, ws)
+                assert G == 1 or G * (hq // 64) <= 256, (hq, B, ns, G)
+                assert (G - 1 + min(B, G - 1)) * hq * 513 * 4 <= ws
+            assert L.tlm_mla_h16_ranges(B, hq, 0) == 1
+    assert L.tlm_mla_h16_ranges(8, 128, 1 << 30) == 128
+    assert L.tlm_mla_h16_ranges(8, 192, 1 << 30) == 85

@@ -547,7 +547,7 @@ int tlm_mla_fp8_launch_segments(const void* q, const void* q_pe, int64_t q_strid
 int tlm_mla_h16_launch(const void* q, const void* q_pe, int64_t q_stride, int64_t q_pe_stride,
                        const void* kv, const void* k_pe, int64_t kv_stride, int64_t kpe_stride,
                        int64_t kv_rows, const int32_t* block_table, const int32_t* seqlens,
-                       void* o, void* ws, int64_t slots, int64_t B, int64_t Hq, int64_t page,
+                       void* o, void* ws, size_t ws_bytes, int64_t B, int64_t Hq, int64_t page,
                        int64_t max_pages, float score_scale, bool bf16, bool o_bf16, void* stream);
 
 // Ranges of the split programs' fp8 path, whatever the program's split count: about 256
@@ -765,7 +765,7 @@ static int mla_run(const char* fn, const void* q, const void* q_pe, int64_t q_st
   if (kv_dtype != TLM_F8E4M3) {
     const int rc = tlm_mla_h16_launch(
         q, q_pe, q_stride, q_pe_stride, kv, k_pe, kv_stride, kpe_stride, kv_rows, block_table, seqlens,
-        o, ws, (int64_t)(ws_bytes / ((size_t)Hq * (MLA_DV + 1) * sizeof(float))), B, Hq, page,
+        o, ws, ws_bytes, B, Hq, page,
         max_pages, sc, q_dtype == TLM_BF16, o_dtype == TLM_BF16, stream);
     if (rc != TLM_EUNSUPPORTED) return rc;
   }

@@ -630,22 +630,29 @@ int mh_launch(const MhArgs& a, hipStream_t st) {
 
 }  // namespace
 
+// Ranges of a decode: one workgroup per CU at most, each holds a CU's whole LDS (one more starts when the first
+// ends and takes as long: 16 x 8,000 tokens of 192 heads 199 us with 258 workgroups, 116 with 255), and
+// as many as the slots (of Hq rows of 513 floats) take: G ranges use at most G - 1 + min(B, G - 1).
+extern "C" int64_t tlm_mla_h16_ranges(int64_t B, int64_t Hq, size_t ws_bytes) {
+  if (B <= 0 || Hq < MH_HEADS) return 0;
+  const int64_t slots = (int64_t)(ws_bytes / ((size_t)Hq * (MH_DV + 1) * sizeof(float)));
+  return std::max<int64_t>(
+      1, std::min(256 / (Hq / MH_HEADS), std::max(slots - B, slots / 2) + 1));
+}
+
 // Balanced decode over a 16-bit cache on validated arguments of the matrix-core shape (tlm_mla.hip: dv 512,
-// dpe 64, Hq a multiple of 64, 16-byte aligned rows). `slots`: slots of Hq rows of 513 floats that ws holds; G
-// ranges use at most G - 1 + min(B, G - 1), and about one workgroup per CU is wanted.
-// TLM_EUNSUPPORTED where every workgroup's own scan of the lengths would cost more than it saves.
+// dpe 64, Hq a multiple of 64, 16-byte aligned rows). TLM_EUNSUPPORTED where every workgroup's own scan of the
+// lengths would cost more than it saves.
 int tlm_mla_h16_launch(const void* q, const void* q_pe, int64_t q_stride, int64_t q_pe_stride,
                        const void* kv, const void* k_pe, int64_t kv_stride, int64_t kpe_stride,
                        int64_t kv_rows, const int32_t* block_table, const int32_t* seqlens, void* o,
-                       void* ws, int64_t slots, int64_t B, int64_t Hq, int64_t page,
+                       void* ws, size_t ws_bytes, int64_t B, int64_t Hq, int64_t page,
                        int64_t max_pages, float score_scale, bool bf16, bool o_bf16, void* stream) {
   // token and cost positions are 32-bit
   if (B > 4096 || max_pages * page > INT32_MAX / 2 ||
       B * (max_pages * page / MH_BN + 1 + MH_PIECE) > INT32_MAX / 2)
     return TLM_EUNSUPPORTED;
-  const int64_t hblocks = Hq / MH_HEADS;
-  const int64_t G = std::max<int64_t>(
-      1, std::min((256 + hblocks - 1) / hblocks, std::max(slots - B, slots / 2) + 1));
+  const int64_t G = tlm_mla_h16_ranges(B, Hq, ws_bytes);
   MhArgs a;
   a.q = (const uint16_t*)q;
   a.q_pe = (const uint16_t*)q_pe;

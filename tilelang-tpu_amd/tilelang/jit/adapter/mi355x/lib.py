@@ -68,6 +68,7 @@ _SIGNATURES = {
                                 c_int64, c_int64, c_void_p, c_void_p, c_void_p] +
                                [c_int64] * 6 + [c_int, c_float, c_void_p, c_int, c_int, c_int,
                                                 c_void_p], c_int),
+    "tlm_mla_h16_ranges": ([c_int64, c_int64, c_size_t], c_int64),
     "tlm_mla_scratch_bytes": ([], c_size_t),
     "tlm_paged_gather": ([c_void_p, c_int64, c_int64, c_void_p, c_void_p, c_void_p, c_void_p,
                           c_int64, c_int64, c_int64, c_void_p], c_int),
