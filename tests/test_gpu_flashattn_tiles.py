@@ -77,9 +77,11 @@ def test_ragged_batch_of_short_sequences():
 
 @pytest.mark.parametrize("B,H,Sq,Skv,ns", [(2, 8, 1, 512, 2), (2, 8, 16, 2048, 4), (2, 8, 128, 1024, 1),
                                            (2, 8, 129, 512, 2), (2, 8, 200, 4096, 8), (3, 3, 40, 2000, 5),
-                                           (1, 1, 128, 4096, 1), (1, 5, 300, 1280, 4)])
+                                           (1, 1, 128, 4096, 1), (1, 5, 300, 1280, 4),
+                                           (4, 32, 64, 2304, 1), (4, 32, 1, 2200, 1)])
 def test_split_inference(B, H, Sq, Skv, ns):
-    """Short query blocks over a key split; fp32 parts merged, lse and partials stored in fp16."""
+    """Short query blocks over a key split, parts on both sides of 1,024 keys; fp32 parts merged, lse and partials
+    stored in fp16."""
     g = torch.Generator(device=DEV).manual_seed(Sq + Skv)
     q = torch.randn(B, Sq, H, 128, generator=g, device=DEV).half()
     k, v = (torch.randn(B, Skv, H, 128, generator=g, device=DEV).half() for _ in range(2))

@@ -958,7 +958,12 @@ int launch_pp(const void* q, const void* k, const void* v, void* o, int B, int S
   const int64_t heads = (int64_t)B * H * (SPLIT ? sp.nsi : 1);
   const int64_t keys = SPLIT ? sp.per_i : sm.cu_q ? S : sm.s_k;
   const FaTiles t = fa_tiles(CAUSAL, heads, S, keys);
-  if (t.nq == 2 || (NT && S > 128))  // NT: a K / V tile is read by one workgroup
+  // NT: a K / V tile is read by one workgroup and its stream is the bound, so the 256-query tile's fewer waves
+  // at work cost nothing once the part is long; on short parts the smaller tile starts and ends earlier.
+  // 128 / 256 queries per workgroup (us a call, 32 heads): 1 x 128 queries, parts of 128 keys 19.6 / 20.9,
+  // 1 x 16, 1,024 keys 28.8 / 29.7, 1 x 128, 1,024 keys 36.9 / 36.6, 2 x 33, 1,280 keys 33.8 / 33.5, 4 x 64,
+  // 4,096 keys 92.7 / 89.6.
+  if (t.nq == 2 || (NT && (S > 128 || keys > 1024)))
     return launch_pp_nq<BF16, CAUSAL, OUT32, SPLIT, NT, 2>(q, k, v, o, B, S, H, Hkv, sc, sm, st, sp,
                                                            t.pairs);
   return launch_pp_nq<BF16, CAUSAL, OUT32, SPLIT, NT, 1>(q, k, v, o, B, S, H, Hkv, sc, sm, st, sp,
