@@ -13,10 +13,10 @@
 // ring by LDS-DMA (NST - 1 tiles in flight, one barrier per tile); the operands of tile t are
 // read from LDS while the MFMAs of tile t - 1 run.
 // The MFMAs take B as the first operand, so a lane holds 4 consecutive columns of one row of C.
-// Measured (us, the 256x256 kernel before -> here): bf16 500 x 4096 x 4096 79 -> 26, 64 x 2048 x 7168
-// B^T 123 -> 12, 1024 x 4096 x 4096 80 -> 40, 2048 x 4096 x 4096 81 -> 64; e4m3 512 x 4096 x 4096
-// 39 -> 20, 16 x 4096 x 4096 (one thread per output before) 1515 -> 8; M 16 B^T 14336 x 4096 (a
-// 64-column strip kernel before) 31.9 -> 20.2, 5.8 TB/s.
+// Measured (us, the 256x256 kernel before -> here): bf16 500 x 4096 x 4096 79 -> 27, 64 x 2048 x 7168
+// B^T 123 -> 11, 1024 x 4096 x 4096 80 -> 40, 2048 x 4096 x 4096 81 -> 66; e4m3 512 x 4096 x 4096
+// 39 -> 22, 16 x 4096 x 4096 (one thread per output before) 1515 -> 9; M 16 B^T 14336 x 4096 (a
+// 64-column strip kernel before) 31.9 -> 22.4, 5.2 TB/s.
 //
 // Split K: every workgroup stores its partial tile (fp32) with write-through stores and counts
 // itself in on the tile's counter; the last to arrive adds the tiles in split order, writes C and
@@ -45,12 +45,11 @@ constexpr uint32_t OOB_OFF = 0xfffffff0u;  // past num_records: the load returns
 constexpr int RSRC3 = 0x00020000;
 
 template <int EL_, bool TRANS_B_, int BM_, int BN_, int WTM_, int WTN_, int BKB_, int NST_,
-          bool NT_ = false, bool WIDE_ = false, bool DUAL_ = false>
+          bool WIDE_ = false, bool DUAL_ = false>
 struct Cfg {
   static constexpr int EL = EL_, BM = BM_, BN = BN_, WTM = WTM_, WTN = WTN_;
   static constexpr int BKB = BKB_;  // bytes of k per tile
   static constexpr int NST = NST_;
-  static constexpr int B_CP = NT_ ? CP_NT : CP_PLAIN;  // cache policy of B's loads
   static constexpr bool TRANS_B = TRANS_B_;
   static constexpr bool FP8 = EL >= EL_E4M3;
   static constexpr bool DUAL = DUAL_;  // two B^T matrices, SwiGLU of the two products
@@ -599,16 +598,14 @@ struct Shape {
 };
 constexpr Shape SHAPES[T_COUNT] = {{32, 64, 256},  {32, 128, 256},  {64, 64, 256},
                                    {64, 64, 256},  {128, 128, 128}, {256, 128, 128}};
-// One workgroup's rows (T32, T32W, T64N: B is read once, with non-temporal loads; 16 x 14336 x 4096
-// B^T from HBM 22.2 -> 20.2 us, 64 rows 27.0 -> 24.6) or several row tiles sharing B in L2. The ring
-// holds at most 64 KB in flight per CU: more stages made the LDS-DMA instructions wait at issue
-// (T128 at 1024 x 4096 x 4096: 39 us with 3 stages, 44 with 4).
+// T32, T32W and T64N hold all rows (B is read once), the others share B in L2 between row tiles. T64N and T64 are
+// one kernel with two cost lines: one row tile, or several. The ring holds at most 64 KB in flight
+// per CU: more stages made the LDS-DMA instructions wait at issue (T128 at 1024 x 4096 x 4096: 39 us with
+// 3 stages, 44 with 4).
 template <int EL, bool TB>
-using C32 = Cfg<EL, TB, 32, 64, 32, 32, 256, 4, true>;
+using C32 = Cfg<EL, TB, 32, 64, 32, 32, 256, 4>;
 template <int EL, bool TB>
-using C32W = Cfg<EL, TB, 32, 128, 32, 32, 256, 3, true>;
-template <int EL, bool TB>
-using C64N = Cfg<EL, TB, 64, 64, 32, 32, 256, 3, true>;
+using C32W = Cfg<EL, TB, 32, 128, 32, 32, 256, 3>;
 template <int EL, bool TB>
 using C64 = Cfg<EL, TB, 64, 64, 32, 32, 256, 3>;
 template <int EL, bool TB>
@@ -621,9 +618,8 @@ struct Plan {
 };
 // The cheapest (tile, split) by a model of the time in us: a launch, its rounds of 256 workgroups
 // times their k-tiles (dearer the more CUs share L2 and memory), and for a split the exchange. The
-// coefficients are a fit to measured times of every tile and split at 355 shapes (M 1-4096,
-// N and K 512-57344); the choice was on average 1.1% (16-bit) and 1.6% (fp8) slower than the
-// best measured one. max_ns 1: no split.
+// coefficients are a fit to measured times of the tiles and splits at M 1-4096, N and K 512-57344.
+// max_ns 1: no split.
 // dual: both matrices of run_swiglu, N columns in all; only_tiles: not the 256 x 256 kernel.
 inline Plan choose(bool fp8, bool trans_b, int64_t M, int64_t N, int64_t K, int max_ns,
                    bool dual = false, bool only_tiles = false) {
@@ -717,7 +713,7 @@ bool run_tiles(Plan p, const void* A, const void* B, void* C, int M, int N, int 
       // keeps the accuracy of the per-output kernel that took them before
       if constexpr (FP8) {
         if (M <= 16) {
-          launch_tile<Cfg<EL, TB, 32, 64, 32, 32, 256, 4, true, true>, OUT>(A, B, C, M, N, K, p.ns, part,
+          launch_tile<Cfg<EL, TB, 32, 64, 32, 32, 256, 4, true>, OUT>(A, B, C, M, N, K, p.ns, part,
                                                                            arrivals, s);
           return true;
         }
@@ -727,7 +723,7 @@ bool run_tiles(Plan p, const void* A, const void* B, void* C, int M, int N, int 
     case T32W:
       if constexpr (!TB) launch_tile<C32W<EL, TB>, OUT>(A, B, C, M, N, K, p.ns, part, arrivals, s);
       return !TB;
-    case T64N: launch_tile<C64N<EL, TB>, OUT>(A, B, C, M, N, K, p.ns, part, arrivals, s); return true;
+    case T64N:
     case T64: launch_tile<C64<EL, TB>, OUT>(A, B, C, M, N, K, p.ns, part, arrivals, s); return true;
     case T128: launch_tile<C128<EL, TB>, OUT>(A, B, C, M, N, K, p.ns, part, arrivals, s); return true;
     case T256: launch_tile<C256<EL, TB>, OUT>(A, B, C, M, N, K, p.ns, part, arrivals, s); return true;
@@ -754,23 +750,20 @@ void run_swiglu(Plan p, const void* A, const void* B, const void* B2, void* C, i
   const uint8_t* const b2 = (const uint8_t*)B2;
   switch (p.tile) {
     case T32W:
-      launch_tile<Cfg<EL, true, 32, 128, 32, 64, 256, 3, true, false, true>, OUT>(
+      launch_tile<Cfg<EL, true, 32, 128, 32, 64, 256, 3, false, true>, OUT>(
           A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
       break;
     case T64N:
-      launch_tile<Cfg<EL, true, 64, 64, 32, 32, 256, 3, true, false, true>, OUT>(
-          A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
-      break;
     case T64:
-      launch_tile<Cfg<EL, true, 64, 64, 32, 32, 256, 3, false, false, true>, OUT>(
+      launch_tile<Cfg<EL, true, 64, 64, 32, 32, 256, 3, false, true>, OUT>(
           A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
       break;
     case T128:
-      launch_tile<Cfg<EL, true, 128, 128, 64, 64, 128, 3, false, false, true>, OUT>(
+      launch_tile<Cfg<EL, true, 128, 128, 64, 64, 128, 3, false, true>, OUT>(
           A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
       break;
     default:
-      launch_tile<Cfg<EL, true, 256, 128, 64, 64, 128, 3, false, false, true>, OUT>(
+      launch_tile<Cfg<EL, true, 256, 128, 64, 64, 128, 3, false, true>, OUT>(
           A, B, C, M, N, K, p.ns, part, arrivals, s, b2);
   }
 }
