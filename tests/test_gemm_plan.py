@@ -7,12 +7,77 @@ from tilelang.jit.adapter.mi355x import lib
 
 PER_THREAD = 2  # hipStreamPerThread
 
+# Calls that reach every tile, whole and split, with remainders in M, N and K, with one row tile and with
+# several: (call, M, N, K, tile rows, tile columns, split). nn / nt: 16-bit row-major B / B^T; fp8: B^T;
+# dual: tlm_gemm_swiglu (N columns of each of its two matrices). test_gpu_gemm_tile.py runs them.
+TILE_CASES = [
+    ("nn", 1, 72, 72, 32, 64, False), ("nn", 1, 72, 776, 32, 64, True),
+    ("nn", 1, 16392, 72, 32, 128, False), ("nn", 1, 3080, 2056, 32, 128, True),
+    ("nn", 33, 72, 72, 64, 64, False), ("nn", 33, 72, 520, 64, 64, True),
+    ("nn", 65, 72, 72, 64, 64, False), ("nn", 65, 72, 1032, 64, 64, True),
+    ("nn", 33, 16392, 264, 128, 128, False), ("nn", 129, 12296, 136, 128, 128, False),
+    ("nn", 65, 8200, 1032, 128, 128, True), ("nn", 200, 4104, 1032, 128, 128, True),
+    ("nn", 129, 16392, 136, 256, 128, False), ("nn", 257, 12296, 136, 256, 128, False),
+    ("nn", 1025, 12296, 136, 256, 256, False),
+    ("nt", 1, 77, 72, 32, 64, False), ("nt", 17, 77, 776, 32, 64, True),
+    ("nt", 33, 77, 72, 64, 64, False), ("nt", 33, 77, 520, 64, 64, True),
+    ("nt", 65, 77, 72, 64, 64, False), ("nt", 65, 77, 1032, 64, 64, True),
+    ("nt", 33, 16397, 264, 128, 128, False), ("nt", 129, 12301, 136, 128, 128, False),
+    ("nt", 65, 8205, 1032, 128, 128, True), ("nt", 200, 4109, 1032, 128, 128, True),
+    ("nt", 129, 16397, 136, 256, 128, False), ("nt", 257, 12301, 136, 256, 128, False),
+    ("nt", 1025, 12301, 136, 256, 256, False),
+    ("fp8", 1, 72, 80, 32, 64, False), ("fp8", 1, 72, 2064, 32, 64, True),
+    ("fp8", 17, 72, 80, 32, 64, False), ("fp8", 20, 72, 2064, 32, 64, True),
+    ("fp8", 33, 72, 80, 64, 64, False), ("fp8", 33, 72, 2064, 64, 64, True),
+    ("fp8", 65, 72, 80, 64, 64, False), ("fp8", 65, 72, 2064, 64, 64, True),
+    ("fp8", 200, 28680, 80, 128, 128, False), ("fp8", 65, 3080, 8208, 128, 128, True),
+    ("fp8", 3000, 72, 8208, 128, 128, True), ("fp8", 1025, 12296, 144, 256, 128, False),
+    ("fp8", 129, 16392, 4112, 256, 256, False),
+    ("dual", 1, 39, 72, 32, 128, False), ("dual", 1, 39, 776, 32, 128, True),
+    ("dual", 33, 39, 72, 64, 64, False), ("dual", 33, 39, 520, 64, 64, True),
+    ("dual", 65, 39, 72, 64, 64, False), ("dual", 65, 39, 1032, 64, 64, True),
+    ("dual", 33, 8199, 264, 128, 128, False), ("dual", 129, 6151, 136, 128, 128, False),
+    ("dual", 65, 4103, 1032, 128, 128, True), ("dual", 200, 2055, 1032, 128, 128, True),
+    ("dual", 129, 8199, 136, 256, 128, False), ("dual", 257, 6151, 136, 256, 128, False),
+]
+# the kernel of one decode step (16 rows, row-major B from 32 MB): K % 16 == 8, ragged strips, uneven ranges
+SKINNY_CASES = [(1, 4104, 4104), (5, 4104, 8200), (16, 14344, 1176), (16, 2056, 8200), (3, 16392, 1032),
+                (16, 6152, 4104)]
+
 
 def plan(M, N, K, dt=lib.F16, trans_b=True, dual=False, stream=None, captured=False):
     out = [ctypes.c_int() for _ in range(3)]
     lib.call("tlm_gemm_plan", M, N, K, dt, int(trans_b), int(dual), stream, int(captured),
              *(ctypes.byref(v) for v in out))
     return tuple(v.value for v in out)
+
+
+@pytest.mark.parametrize("call,M,N,K,rows,cols,split", TILE_CASES)
+def test_tile_cases_take_their_tile(call, M, N, K, rows, cols, split):
+    for dt in (lib.F8E4M3, lib.F8E5M2) if call == "fp8" else (lib.F16, lib.BF16):
+        r, c, ns = plan(M, N, K, dt, trans_b=call != "nn", dual=call == "dual")
+        assert (r, c, ns > 1) == (rows, cols, split)
+
+
+def test_tile_cases_cover_every_tile():
+    """Every (tile, split or not) that any call of a grid of shapes takes is among the cases."""
+    seen = {(c[0], *c[4:]) for c in TILE_CASES}
+    for M in (1, 16, 17, 33, 64, 65, 128, 200, 257, 500, 1000, 2048, 4096):
+        for N in (72, 520, 1032, 2056, 4104, 8200, 14336, 28680):
+            for K in (72, 264, 1032, 2064, 4096, 8208, 14336):
+                for call in ("nn", "nt", "fp8", "dual"):
+                    if call == "fp8" and K % 16:
+                        continue
+                    r, c, ns = plan(M, N, K, lib.F8E4M3 if call == "fp8" else lib.F16,
+                                    trans_b=call != "nn", dual=call == "dual")
+                    if (r, c) == (16, 128) or (call == "dual" and c == 256):
+                        continue  # the decode kernel, or three calls
+                    assert (call, r, c, ns > 1) in seen, (call, M, N, K, r, c, ns)
+
+
+@pytest.mark.parametrize("M,N,K", SKINNY_CASES)
+def test_skinny_cases_take_the_decode_kernel(M, N, K):
+    assert plan(M, N, K, trans_b=False)[:2] == (16, 128)
 
 
 SPLIT_CALLS = [dict(M=16, N=14336, K=4096, trans_b=False), dict(M=16, N=4096, K=14336, trans_b=False),

@@ -22,7 +22,9 @@ REPEAT = 4
     ("gemm_rowmajor_b", lambda: programs.matmul(512, 768, 1024, 256, 256, 64), -1),
     ("gemm_bt_bf16", lambda: programs.matmul(300, 520, 256, 256, 256, 64, "bfloat16",
                                              "bfloat16", trans_b=True), -1),
-    ("gemm_skinny", lambda: programs.matmul(16, 4096, 1024, 16, 64, 64), -1),
+    ("gemm_16_rows", lambda: programs.matmul(16, 4096, 1024, 16, 64, 64), -1),
+    ("gemm_skinny", lambda: programs.matmul(16, 8192, 4096, 16, 64, 64), -1),
+    ("gemm_split_tiles", lambda: programs.matmul(200, 4096, 1024, 128, 128, 64), -1),
     ("gemm_fp8", lambda: programs.matmul_fp8(512, 512, 1024, 128, 128, 64, "e4m3_float8",
                                              two_acc=True), -1),
     ("flashattn_causal_paired", lambda: programs.flashattn(2, 4, 1100, 128, True), -1),

@@ -62,8 +62,8 @@ def test_gemm_trans_b_and_out_dtypes(M, N, K, out):
 
 @pytest.mark.parametrize("M,N,K", [(5, 100, 96), (16, 1000, 520), (3, 4104, 4096)])
 def test_gemm_skinny_nonfinite_column_stays_in_its_column(M, N, K):
-    """The skinny kernel reads whole 64-column strips of B; in the last, ragged strip the columns
-    past N hold the next row's leading values. A NaN / inf column 0 of B must reach column 0 of C
+    """The kernels read whole strips of 64 or 128 columns of B (5 x 100 is a tile, 3 x 4104 the kernel of one decode
+    step); in the last, ragged strip the columns past N hold the next row's leading values. A NaN / inf column 0 of B must reach column 0 of C
     only: every other column matches the oracle."""
     g = torch.Generator().manual_seed(M + N + K)
     a = (torch.rand(M, K, generator=g) * 2 - 1).half()
@@ -78,7 +78,7 @@ def test_gemm_skinny_nonfinite_column_stays_in_its_column(M, N, K):
 
 
 def test_gemm_skinny_split_repeatable():
-    """M <= 16 with row-major B splits K over several workgroups per column strip; the partial
+    """M <= 16 with 32 MB of row-major B splits K over several workgroups per column strip; the partial
     tiles are summed in split order by whichever workgroup arrives last, and the arrival counters
     are left at zero: reruns are bitwise equal, also after calls of other shapes in between."""
     g = torch.Generator().manual_seed(21)
@@ -99,8 +99,7 @@ def test_gemm_skinny_split_repeatable():
 @pytest.mark.parametrize("M,N,K", [(16, 4096, 14336), (5, 1000, 2056), (1, 64, 8192),
                                    (16, 520, 4104)])
 def test_gemm_skinny_bt_split(M, N, K):
-    """M <= 16 with B^T and few 64-column strips splits K over several workgroups per strip
-    (one per CU in all); the partial tiles meet in split order: parity with the oracle, and
+    """M <= 16 with B^T and few columns splits K over several workgroups per 32 x 64 tile; the partial tiles meet in split order: parity with the oracle, and
     reruns (with other split calls in between) are bitwise equal."""
     g = torch.Generator().manual_seed(M + N + K)
     a = (torch.rand(M, K, generator=g) * 2 - 1).half()
@@ -117,8 +116,8 @@ def test_gemm_skinny_bt_split(M, N, K):
 
 
 def test_gemm_skinny_concurrent_streams():
-    """Each stream owns one workspace slot of the split skinny kernel (4 per device); further
-    streams take the unsplit kernel. Six streams run skinny GEMMs at the same time, twice over,
+    """Each stream owns one workspace slot of the split calls of 16 rows or fewer (4 per device); further
+    streams run unsplit. Six streams run such GEMMs at the same time, twice over,
     and every result matches the oracle."""
     g = torch.Generator().manual_seed(22)
     shapes = [(16, 4096, 4096), (8, 6144, 2048), (16, 2048, 8192), (1, 4096, 4096),

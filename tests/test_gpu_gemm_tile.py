@@ -1,6 +1,6 @@
-"""GPU parity of the tiles between one decode step and a whole prompt batch (tlm_gemm_tile.h): sizes
-at the edges of every tile (32, 64, 128, 256 rows; 64 and 128 columns; 64- and 128-value k-tiles),
-remainders on each axis, and K splits, against the fp64 product of the same inputs.
+"""GPU parity of the tiles between one decode step and a whole prompt batch (tlm_gemm_tile.h): every tile, whole
+and split over K, with remainders on each axis (TILE_CASES, whose tiles test_gemm_plan.py asserts), and a list of
+mixed shapes, against the fp64 product of the same inputs.
 
 Tolerance: fp32 sums of K products with |partial sums| <= s err by at most K ulp(s) / 2; here the
 relative 2-norm error stays below 4 sqrt(K) 2^-24, plus half an ulp of the output type (2^-9 bf16,
@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from conftest import PKG
+from test_gemm_plan import SKINNY_CASES, TILE_CASES
 from tilelang.jit.adapter.mi355x import ops
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +33,42 @@ def _run(M, N, K, dt, out, trans_b, seed=0, scale=1.0):
     ops.gemm(a, b, c, trans_b=trans_b)
     bd = b.double()
     return c, a.double() @ (bd.T if trans_b else bd)
+
+
+def _swiglu(M, N, K, dt, shift=0):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g, device=DEV).to(dt)
+    bg, bu = ((torch.randn(N * K + 1, generator=g, device=DEV) * K ** -0.5).to(dt)[shift:shift + N * K].view(N, K)
+              for _ in range(2))
+    h = torch.full((M, N), float("nan"), dtype=dt, device=DEV)
+    ops.gemm_swiglu(a, bg, bu, h)
+    gate, up = a.double() @ bg.double().T, a.double() @ bu.double().T
+    assert _rel(h, up * gate * torch.sigmoid(gate)) < 3 * ULP[dt]
+
+
+OUTS = {"nn": [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)],
+        "nt": [(torch.float16, torch.float16), (torch.bfloat16, torch.float32)],
+        "fp8": [(torch.float8_e4m3fn, torch.float32), (torch.float8_e5m2, torch.float32)],
+        "dual": [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16)]}
+
+
+@pytest.mark.parametrize("call,M,N,K,rows,cols,split", TILE_CASES)
+def test_every_tile(call, M, N, K, rows, cols, split):
+    for dt, out in OUTS[call]:
+        if call == "dual":
+            _swiglu(M, N, K, dt)
+            continue
+        c, exp = _run(M, N, K, dt, out, call != "nn")
+        low_bits = 5e-5 if call == "fp8" and M > 16 else 0
+        assert _rel(c, exp) < 4 * K ** 0.5 * 2.0 ** -24 + ULP[out] + low_bits
+
+
+@pytest.mark.parametrize("M,N,K", SKINNY_CASES)
+def test_decode_kernel(M, N, K):
+    """One decode step on 32 MB of row-major B or more."""
+    for dt, out in OUTS["nn"]:
+        c, exp = _run(M, N, K, dt, out, False)
+        assert _rel(c, exp) < 4 * K ** 0.5 * 2.0 ** -24 + ULP[out]
 
 
 SHAPES = [(17, 64, 64), (32, 136, 200), (33, 64, 4096), (64, 2048, 1000), (65, 520, 2048),
@@ -125,15 +162,8 @@ def test_gemm_split_tiles_repeat_and_replay():
 def test_gemm_swiglu(M, N, K, dt):
     """up * silu(gate) of two products, each rounded to the dtype first; K 60 and a weight that is not
     16-byte aligned run as three calls. Three roundings of half an ulp each."""
-    g = torch.Generator(device=DEV).manual_seed(M + N + K)
-    a = torch.randn(M, K, generator=g, device=DEV).to(dt)
-    w = [(torch.randn(N * K + 1, generator=g, device=DEV) * K ** -0.5).to(dt) for _ in range(2)]
     for shift in (0, 1) if M <= 33 else (0,):
-        bg, bu = (x[shift:shift + N * K].view(N, K) for x in w)
-        h = torch.full((M, N), float("nan"), dtype=dt, device=DEV)
-        ops.gemm_swiglu(a, bg, bu, h)
-        gate, up = a.double() @ bg.double().T, a.double() @ bu.double().T
-        assert _rel(h, up * gate * torch.sigmoid(gate)) < 3 * ULP[dt]
+        _swiglu(M, N, K, dt, shift)
 
 
 DECODE_SLOTS = """

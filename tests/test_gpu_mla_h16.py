@@ -61,7 +61,8 @@ def _check(out, exp, lens, dt):
 
 
 @pytest.mark.parametrize("lens", [[1], [64], [65, 0, 63], [3000], [500, 4000, 1, 128, 0, 2000, 77, 640],
-                                  [33] * 40, [0, 0, 5], [1300] * 16])
+                                  [33] * 40, [0, 0, 5], [1300] * 16,
+                                  [31, 32, 33, 511, 512, 513, 16384]])
 @pytest.mark.parametrize("H,page,dt", [(128, 64, torch.bfloat16), (64, 16, torch.float16),
                                        (192, 100, torch.bfloat16), (256, 128, torch.float16)])
 def test_lengths_and_heads(lens, H, page, dt):

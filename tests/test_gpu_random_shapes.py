@@ -1,5 +1,5 @@
 """GPU parity over seeded random shapes for the tiled MFMA kernels (16x16 operand layouts, LDS
-swizzles, edge masking): GEMM (both B layouts, fp16 / bf16, ragged M, N, K, skinny M <= 16), FP8 GEMM and
+swizzles, edge masking): GEMM (both B layouts, fp16 / bf16, ragged M, N, K, M <= 16), FP8 GEMM and
 FlashAttention (causal or not, grouped K/V heads, head dim 64 and 128, ragged S), and the other
 attention layouts over random shapes and head dims 8-256: head-major with independent query and
 key lengths, variable length, split-KV inference with its partials. Each case prints its shape
@@ -58,8 +58,8 @@ def _skinny_cases(n, seed):
 
 @pytest.mark.parametrize("M,N,K,trans_b,dt", _skinny_cases(16, seed=77))
 def test_gemm_skinny_random(M, N, K, trans_b, dt):
-    """M <= 16 takes the skinny kernels: A staged in LDS for row-major B and K <= 4096, A read
-    per block otherwise (K past 4096, B^T); ragged N and K not a multiple of 32 included."""
+    """M <= 16 on the 32-row tiles, whole and split over K (B below 32 MB; the kernel of one decode step is
+    test_gpu_gemm_tile.py's); ragged N and K not a multiple of 32 included."""
     test_gemm_random(M, N, K, trans_b, dt)
 
 
