@@ -5,15 +5,14 @@
 // heads a multiple of 64.
 //
 // What bounds it: fixed costs at small batches, the tile's own chain at large ones. 8 sequences of
-// 500 .. 4,000 tokens, 128 heads (bf16): 25.0 us and 8.0 us for the combine, where the split kernel that
+// 500 .. 4,000 tokens, 128 heads (bf16): 26.0 us and 8.2 us for the combine, where the split kernel that
 // it replaced took 67.2 and 14.7; 20.7 MB of cache rows would take 3.1 us. Inside a workgroup 1.6 us go to the
 // scan, 5 to the block table and Q, 2.6 to the first tile and 2 to 4 to the partial rows (33 MB of fp32 for
-// 128 ranges, written and read again); the rest is the launch. 16 x 4,000 .. 8,000 tokens: 61 us, of which a
-// 32-token tile takes 1.8 with the next ones already there. It has 1,100 cycles of MFMA issue per SIMD
+// 128 ranges, written and read again); the rest is the launch. 16 x 4,000 .. 8,000 tokens: 64.6 us, of which a
+// 32-token tile takes 1.9 with the next ones already there. It has 1,100 cycles of MFMA issue per SIMD
 // and 1,450 of LDS reads per CU (K and V^T operands, 140 KB); leaving out the loads or the MFMAs, or
 // taking the rows from L2, changes the kernel's time by less than 5 %: the chain read, multiply, exchange,
-// softmax, barrier is what remains, with two waves per SIMD to overlap it. Joining S^T of a tile and
-// O^T of the one before it into one stretch with one barrier less measured the same (61.9 us).
+// softmax, barrier is what remains, with two waves per SIMD to overlap it.
 //
 //   * Partition: sequence b costs its 32-token tiles plus MH_PIECE for fetching Q and writing rows; the cost
 //     line of the batch is cut into G equal ranges, one per workgroup and 64 heads. A sequence
@@ -21,16 +20,16 @@
 //     normalised O and log2 sum-exp) that mla_h16_combine merges. Every workgroup finds its own range
 //     from the lengths (a block scan), so there is no preparing launch.
 //   * Wave (hg, th, dh): 32 heads (hg). For S^T, 16 of the tile's tokens (th) over one half of the 576 dims
-//     (Q in 72 registers; all of Q would take 144 and spill): the wave and its partner swap the half
-//     scores of 16 heads each (16 KB of LDS traffic a tile) and finish 16 tokens x 16 heads. P^T goes
-//     through LDS, and the wave multiplies V^T rows 128 (2 th + dh) .. + 127 of all 32 tokens. The earlier
-//     kernel split the 576 dims four ways, exchanged 160 KB of partial scores per 32 tokens and repeated
-//     the softmax in four waves.
+//     (Q in 72 registers; all of Q would take 144 and spill). The four waves of a head group then exchange their
+//     partial sums (12 KB of LDS traffic a tile) so that each finishes 32 tokens x 8 heads, whose maximum it
+//     has in its own lanes. P^T goes through LDS, and the wave multiplies V^T rows 128 (2 th + dh) .. + 127 of
+//     all 32 tokens. The earlier kernel split the 576 dims four ways, exchanged 160 KB of partial scores per 32
+//     tokens and repeated the softmax in four waves.
 //   * Softmax against the running maximum of each head, so that the largest weight is exactly 1 in 16 bits
-//     and a piece may start with tiles that score -inf: the two token halves' maxima meet in LDS, and O is
-//     rescaled where a head's maximum rose. Against a reference that only the first tile set (kept until some P left
-//     the 16-bit range) that is one barrier more per tile: 16 x 4,000 .. 8,000 tokens 66.4 -> 72.4 us, 8 x
-//     500 .. 4,000 31.5 -> 32.3; its error was larger (2.0e-3 of fp64 against 1.9e-3 here, bf16).
+//     and a piece may start with tiles that score -inf. O is rescaled beside the MFMAs. Against a reference that
+//     only the first tile set (kept until some P left the 16-bit range, error 2.0e-3 of fp64 instead of 1.9e-3
+//     in bf16): 16 x 4,000 .. 8,000 tokens 66.4 -> 69.6 us, 8 x 500 .. 4,000 31.4 -> 31.8. Finishing 16 tokens x
+//     16 heads per wave, the halves' maxima meeting in LDS behind a fourth barrier: 72.2 and 32.3.
 //   * Tiles stream through a four-stage LDS ring by LDS-DMA (latent rows one 1 KB instruction per token, rope
 //     rows 8 tokens per instruction). The cache rows of 512 tokens at a time are looked up half a block
 //     ahead into an LDS table. 16-byte chunk c of token r sits at c ^ f(r), f(r) = 2 (r % 8) + r / 8 % 2:
@@ -51,13 +50,14 @@ constexpr int MH_PIECE = 6;                     // cost of a piece beside its ti
 constexpr int MH_LAT = MH_BN * MH_DV * 2;       // bytes of a tile's latent rows
 constexpr int MH_STAGE = MH_LAT + MH_BN * MH_DPE * 2;
 constexpr int MH_NST = 4;
-// Per wave 1 KB: the partner's half scores ([64 lanes] f32x4) and, once the wave has read them, its P^T
-// block ([4 lane groups][16 heads][4 tokens] 16-bit) and its 16 maxima / row sums.
-constexpr int MH_P = MH_NST * MH_STAGE, MH_BOX = 1024, MH_BOX_X = 512;
+// Per wave 1.5 KB: the half scores of its 8 heads that the three other waves of its 32 heads bring (3 x 512
+// bytes) and, once it has read them, its P^T block (512 bytes) and 8 factors, row sums and maxima.
+constexpr int MH_P = MH_NST * MH_STAGE, MH_BOX = 1536, MH_BOX_X = 512;
 constexpr int MH_TBL = 512;                     // tokens of a look-up block; two blocks
 constexpr int MH_TBL_TILES = MH_TBL / MH_BN;
+constexpr uint32_t MH_NO_ROW = 0xffffffffu;  // (rows are 1 KB or more: memory ends before the 2^32nd)
 constexpr int MH_ROWS = MH_P + 8 * MH_BOX;
-constexpr int MH_SMEM = MH_ROWS + 2 * MH_TBL * 8;
+constexpr int MH_SMEM = MH_ROWS + 2 * MH_TBL * 4;
 static_assert(MH_SMEM <= 160 * 1024, "LDS");
 
 struct MhArgs {
@@ -140,6 +140,9 @@ TLM_DEV void mh_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
+}
+TLM_DEV float mh_ror8(float x) {  // of lane l ^ 8
+  return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), 0x128, 0xf, 0xf, false));
 }
 TLM_DEV uint32_t mh_lds(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
@@ -273,15 +276,27 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
   const int vt = 4 * g + (jl >> 2);
   const uint32_t v_a = s0 + (uint32_t)(vt * (MH_DV * 2) + 256 * w +
                                        16 * (((jl & 3) >> 1) ^ f_swz(vt)) + 8 * (jl & 1));
-  // boxes: own, the partner's (the same tokens, the other dims), and those of the wave's head group
-  const uint32_t box = s0 + MH_P + (uint32_t)wave * MH_BOX;
-  const uint32_t box_partner = s0 + MH_P + (uint32_t)(wave ^ 1) * MH_BOX;
-  const uint32_t box_hg = s0 + MH_P + (uint32_t)(4 * hg) * MH_BOX;
-  // P^T block of wave 2 th + dh: token 16 th + 4 g + i, head 16 dh + jl of the group's 32
-  const uint32_t p_off = (uint32_t)(g * 128 + jl * 8);
-  auto x_addr = [&](int t2, int hh) {
-    return box_hg + (uint32_t)((2 * t2 + hh) * MH_BOX + MH_BOX_X + jl * 4);
-  };
+  // Exchange (the boxes of the four waves of a head group). Wave w finishes heads 8 w .. + 7 of the group's 32:
+  // lane (g, jl) head 8 w + jl % 8 and, where jl / 8 == dh, the wave's own 16 tokens 4 g + i, else the other
+  // half's. Block 0 of its box comes from the wave of the other dims (the own quarter stays in
+  // registers), blocks 1 and 2 from the waves of the other tokens; the ^ 8 and ^ 2 keep the two
+  // halves jl / 8 of an access on different banks.
+  const int oct = jl >> 3, pos = g * 8 + (jl & 7);
+  const bool own = oct == dh;
+  const int t_fin = own ? th : 1 - th;  // token half that the lane finishes
+  const uint32_t box_hg = s0 + MH_P + (uint32_t)(4 * hg) * MH_BOX, box = box_hg + (uint32_t)w * MH_BOX;
+  const uint32_t put_dims = box_hg + (uint32_t)((w ^ 1) * MH_BOX + (pos ^ 8 * (dh ^ 1)) * 16);
+  const uint32_t put_toks = box_hg + (uint32_t)((2 * (1 - th) + oct) * MH_BOX + (1 + dh) * 512 +
+                                                (pos ^ 8 * (oct ^ dh ^ 1)) * 16);
+  const uint32_t get_1 = box + (uint32_t)((own ? 0 : 512) + (pos ^ 8 * (own ? dh : dh ^ 1)) * 16);
+  const uint32_t get_2 = box + (uint32_t)(1024 + (pos ^ 8 * dh) * 16);
+  // P^T: token half t2, lane group, head, 4 tokens; the reader takes head jl of the group's tiles hh (+ 2 hh boxes)
+  const uint32_t put_p = box + (uint32_t)(t_fin * 256 + (g ^ 2 * (t_fin ^ dh)) * 64 + (jl & 7) * 8);
+  const uint32_t get_p0 = box_hg + (uint32_t)(oct * MH_BOX + (g ^ 2 * oct) * 64 + (jl & 7) * 8);
+  const uint32_t get_p1 = box_hg + (uint32_t)(oct * MH_BOX + 256 + (g ^ 2 * (oct ^ 1)) * 64 + (jl & 7) * 8);
+  // one value per head (every lane of a head writes the same)
+  const uint32_t put_x = box + (uint32_t)(MH_BOX_X + (jl & 7) * 4);
+  const uint32_t get_x = box_hg + (uint32_t)(oct * MH_BOX + MH_BOX_X + (jl & 7) * 4);
   const uint32_t row_tbl = s0 + MH_ROWS;
   const bool rope_wave = wave < 4;
 
@@ -302,36 +317,30 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
     auto entry = [&](int k) { return token(k) < L ? bt[token(k) / a.page] : -1; };
     auto put_row = [&](int k, int e) {
       const int64_t row = (int64_t)e * a.page + token(k) % a.page;
-      const int64_t v = token(k) < L && e >= 0 && row < a.kv_rows ? row : -1;
-      ds_put64(row_tbl + (uint32_t)(((k & 1) * MH_TBL + tid) * 8),
-               u32x2{(uint32_t)v, (uint32_t)((uint64_t)v >> 32)});
+      const bool ok = token(k) < L && e >= 0 && row < a.kv_rows && row < MH_NO_ROW;
+      ds_put32(row_tbl + (uint32_t)(((k & 1) * MH_TBL + tid) * 4), ok ? (uint32_t)row : MH_NO_ROW);
     };
     // ---- loads of tile i of the piece: the wave's four latent rows, and eight rope rows (waves 0 .. 3)
     auto issue = [&](int i) __attribute__((always_inline)) {
-      u32x2 rv;  // lane l < 32: row of token l of the tile
-      {
-        const uint32_t ad = row_tbl + (uint32_t)((i & (2 * MH_TBL_TILES - 1)) * MH_BN * 8 + (lane & 31) * 8);
-        asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(rv) : "v"(ad) : "memory");
-      }
+      // lane l < 32: row of token l of the tile
+      const uint32_t rv = ds_get32(row_tbl + (uint32_t)((i & (2 * MH_TBL_TILES - 1)) * MH_BN * 4 + (lane & 31) * 4));
       const int stage = i & (MH_NST - 1);
       uint8_t* const dst = smem + stage * MH_STAGE;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const uint32_t rl = __builtin_amdgcn_readlane(rv[0], 4 * wave + k);
-        const uint32_t rh = __builtin_amdgcn_readlane(rv[1], 4 * wave + k);
-        const int64_t ri = (int64_t)(((uint64_t)rh << 32) | rl);
-        const bool ok = ri >= 0;  // uniform; rows outside the pool and past the length read as zeros
+        const uint32_t ri = __builtin_amdgcn_readlane(rv, 4 * wave + k);
+        const bool ok = ri != MH_NO_ROW;  // uniform; rows outside the pool and past the length read as zeros
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(a.kv + (ok ? ri : 0) * a.kvs_b), (short)0, ok ? MH_DV * 2 : 0, 0x00020000);
+            (void*)(a.kv + (int64_t)(ok ? ri : 0) * a.kvs_b), (short)0, ok ? MH_DV * 2 : 0, 0x00020000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             rs, (__attribute__((address_space(3))) void*)(dst + (4 * wave + k) * (MH_DV * 2)), 16,
             16 * (lane ^ f_swz(4 * wave + k)), 0, 0, 0);
       }
       if (rope_wave) {
         const int t = 8 * wave + (lane >> 3);
-        const uint32_t rl = (uint32_t)__shfl((int)rv[0], t, 64), rh = (uint32_t)__shfl((int)rv[1], t, 64);
-        const int64_t ri = (int64_t)(((uint64_t)rh << 32) | rl);
-        const uint8_t* const src = ri >= 0 ? a.k_pe + ri * a.kpes_b : (const uint8_t*)mh_zero_row;
+        const uint32_t ri = (uint32_t)__shfl((int)rv, t, 64);
+        const uint8_t* const src =
+            ri != MH_NO_ROW ? a.k_pe + (int64_t)ri * a.kpes_b : (const uint8_t*)mh_zero_row;
         __builtin_amdgcn_global_load_lds(
             (const __attribute__((address_space(1))) void*)(src + 16 * ((lane & 7) ^ ((t >> 1) & 7))),
             (__attribute__((address_space(3))) void*)(dst + MH_LAT + 1024 * wave), 16, 0, 0);
@@ -367,7 +376,7 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
     f32x4 oacc[8][2];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) oacc[dt][0] = oacc[dt][1] = f32x4{};
-    float m[2] = {-INFINITY, -INFINITY}, l = 0.f;  // m of both head tiles, l of the wave's own
+    float m = -INFINITY, l = 0.f;  // of the head that the lane finishes (l: of its tokens)
 
     for (int t = 0; t < n; ++t) {
       const int left = min(MH_NST - 2, n - 1 - t);  // later tiles whose loads may stay in flight
@@ -387,11 +396,10 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
       if (t + MH_NST - 1 < n) issue(t + MH_NST - 1);
       const uint32_t so = (uint32_t)((t & (MH_NST - 1)) * MH_STAGE);
 
-      // ---- S^T = K Q^T: half the dims for 32 heads, then the sums of 16
-      f32x4 s;
+      // ---- S^T = K Q^T: half the dims of 16 tokens x 32 heads, then the sums of 32 tokens x 8 heads
+      f32x4 h[2] = {f32x4{}, f32x4{}};
       auto scores = [&](auto dc) __attribute__((always_inline)) {
         constexpr int DH = decltype(dc)::value, DEPTH = 6;
-        f32x4 h[2] = {f32x4{}, f32x4{}};
         u32x4 op[DEPTH];
         const uint32_t ka = k_a + so, ra = r_a + so;
         auto read = [&](auto ic) __attribute__((always_inline)) {
@@ -413,115 +421,120 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
 #pragma unroll
           for (int hh = 0; hh < 2; ++hh) h[hh] = mh_mma<BF16>(op[n_ % DEPTH], qreg[hh][n_], h[hh]);
         });
-        ds_put_acc(box_partner + 16 * lane, h[1 - DH]);
-        mh_barrier();
-        u32x4 in;
-        ds_b128<0>(in, box + 16 * lane);
-        lgkm_wait<0>();
-        landed(in);
-        // the lower dims' half first in both waves of the pair
-        s = DH == 0 ? h[0] + __builtin_bit_cast(f32x4, in) : __builtin_bit_cast(f32x4, in) + h[1];
       };
       if (dh == 0)
         scores(std::integral_constant<int, 0>{});
       else
         scores(std::integral_constant<int, 1>{});
-      // lane: tokens 16 th + 4 g + i of the tile, head 16 dh + jl
-      const int tok = (t0 + t) * MH_BN + 16 * th + 4 * g;
+      const f32x4 h_own = th ? h[1] : h[0], h_oth = th ? h[0] : h[1];
+      if (!own) ds_put_acc(put_dims, h_own);
+      ds_put_acc(put_toks, h_oth);
+      mh_barrier();
+      f32x4 s;
+      {
+        u32x4 in1, in2;
+        ds_b128<0>(in1, get_1);
+        ds_b128<0>(in2, get_2);
+        lgkm_wait<0>();
+        landed(in1);
+        landed(in2);
+        s = __builtin_bit_cast(f32x4, in1) + (own ? h_own : __builtin_bit_cast(f32x4, in2));
+      }
+      // the first V^T operands: they arrive while the weights are made
+      constexpr int VDEPTH = 5;
+      u32x2 vl[VDEPTH], vh[VDEPTH];
+      const uint32_t va = v_a + so;
+      auto read_v = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int dt = decltype(ic)::value;
+        if constexpr (dt < 8) {
+          ds_tr16<0>(vl[dt % VDEPTH], va ^ (32 * dt));
+          ds_tr16<16 * MH_DV * 2>(vh[dt % VDEPTH], va ^ (32 * dt));
+        }
+      };
+      unroll<0, VDEPTH - 1>(read_v);
+      // ---- weights against the running maximum of the lane's head
+      const int tok = (t0 + t) * MH_BN + 16 * t_fin + 4 * g;
 #pragma unroll
       for (int i = 0; i < 4; ++i) s[i] = tok + i < L ? s[i] * a.c : -INFINITY;
-      // the running maximum, over both token halves
       {
         float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-        mx = xhalf_max(xrow_max(mx));
-        if (g == 0) ds_put32(x_addr(th, dh), __float_as_uint(mx));
-      }
-      mh_barrier();
-      uint32_t mt[2][2];  // the tile's maxima: [head tile][token half]
-      asm volatile(
-          "ds_read_b32 %0, %4\n\tds_read_b32 %1, %4 offset:%5\n\tds_read_b32 %2, %4 offset:%6\n\t"
-          "ds_read_b32 %3, %4 offset:%7\n\ts_waitcnt lgkmcnt(0)"
-          : "=&v"(mt[0][0]), "=&v"(mt[1][0]), "=&v"(mt[0][1]), "=&v"(mt[1][1])
-          : "v"(x_addr(0, 0)), "i"(MH_BOX), "i"(2 * MH_BOX), "i"(3 * MH_BOX)
-          : "memory");
-      float al[2];
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh) {
-        const float y = fmaxf(m[hh], fmaxf(__uint_as_float(mt[hh][0]), __uint_as_float(mt[hh][1])));
-        al[hh] = y == -INFINITY ? 1.f : fast_exp2(m[hh] - y);
-        m[hh] = y;
-      }
-      {
-        const float mo = dh ? m[1] : m[0];
-        const float mm = mo == -INFINITY ? 0.f : mo;
+        mx = fmaxf(mx, mh_ror8(mx));
+        mx = fmaxf(m, xhalf_max(xrow_max(mx)));
+        const float al = mx == -INFINITY ? 1.f : fast_exp2(m - mx);
+        const float mm = mx == -INFINITY ? 0.f : mx;
+        m = mx;
         f32x4 p;
 #pragma unroll
         for (int i = 0; i < 4; ++i) p[i] = fast_exp2(s[i] - mm);
-        l = l * (dh ? al[1] : al[0]) + ((p[0] + p[1]) + (p[2] + p[3]));
-        ds_put64(box + p_off, u32x2{HH::pack(p[0], p[1]), HH::pack(p[2], p[3])});
+        l = l * al + ((p[0] + p[1]) + (p[2] + p[3]));
+        ds_put64(put_p, u32x2{HH::pack(p[0], p[1]), HH::pack(p[2], p[3])});
+        ds_put32(put_x, __float_as_uint(al));
       }
+      mh_barrier();  // every wave's P^T and factors are in LDS, and this wave's V^T operands have landed
 #pragma unroll
-      for (int hh = 0; hh < 2; ++hh)
-        if (__builtin_amdgcn_ballot_w64(!(al[hh] == 1.f))) {  // rarely after a piece's first tiles
-#pragma unroll
-          for (int dt = 0; dt < 8; ++dt) oacc[dt][hh] *= al[hh];
-        }
-      mh_barrier();  // every wave's P^T is in LDS
+      for (int i = 0; i < VDEPTH - 1; ++i) {
+        landed(vl[i]);
+        landed(vh[i]);
+      }
 
       // ---- O^T += V^T P^T: dims 128 w .. of the wave's 32 heads over the tile's 32 tokens
-      u32x2 pb[2][2];  // [head tile][token half]
-      const uint32_t pa = box_hg + p_off, va = v_a + so;
-      unroll<0, 4>([&](auto ic) __attribute__((always_inline)) {
-        constexpr int n_ = decltype(ic)::value, hh = n_ / 2, t2 = n_ % 2;
-        ds_b64<(2 * t2 + hh) * MH_BOX>(pb[hh][t2], pa);
+      u32x2 pb[2][2], al;  // [head tile][token half]; the factors of the two head tiles
+      asm volatile("ds_read2st64_b32 %0, %1 offset1:%2" : "=v"(al) : "v"(get_x), "i"(2 * MH_BOX / 256) : "memory");
+      unroll<0, 2>([&](auto ic) __attribute__((always_inline)) {
+        constexpr int hh = decltype(ic)::value;
+        ds_b64<2 * hh * MH_BOX>(pb[hh][0], get_p0);
+        ds_b64<2 * hh * MH_BOX>(pb[hh][1], get_p1);
       });
-      {
-        constexpr int DEPTH = 5;  // with P^T's 4 reads 14 in flight: lgkmcnt counts to 15
-        u32x2 vl[DEPTH], vh[DEPTH];
-        auto read = [&](auto ic) __attribute__((always_inline)) {
-          constexpr int dt = decltype(ic)::value;
-          if constexpr (dt < 8) {
-            ds_tr16<0>(vl[dt % DEPTH], va ^ (32 * dt));
-            ds_tr16<16 * MH_DV * 2>(vh[dt % DEPTH], va ^ (32 * dt));
-          }
-        };
-        unroll<0, DEPTH - 1>(read);
-        unroll<0, 8>([&](auto ic) __attribute__((always_inline)) {
-          constexpr int dt = decltype(ic)::value;
-          read(std::integral_constant<int, dt + DEPTH - 1>{});
-          constexpr int ahead = 2 * (7 - dt < DEPTH - 1 ? 7 - dt : DEPTH - 1);
-          lgkm_wait<ahead>();
-          landed(vl[dt % DEPTH]);
-          landed(vh[dt % DEPTH]);
-          if constexpr (dt == 0) {
-            landed(pb[0][0]);
-            landed(pb[0][1]);
-            landed(pb[1][0]);
-            landed(pb[1][1]);
-          }
-          const u32x4 v = {vl[dt % DEPTH][0], vl[dt % DEPTH][1], vh[dt % DEPTH][0], vh[dt % DEPTH][1]};
+      lgkm_wait<0>();
+      landed(al);
 #pragma unroll
-          for (int hh = 0; hh < 2; ++hh) {
-            const u32x4 p = {pb[hh][0][0], pb[hh][0][1], pb[hh][1][0], pb[hh][1][1]};
-            oacc[dt][hh] = mh_mma<BF16>(v, p, oacc[dt][hh]);
-          }
-        });
+      for (int hh = 0; hh < 2; ++hh) {
+        landed(pb[hh][0]);
+        landed(pb[hh][1]);
       }
+      // O's rescale of d-tile dt + 1 runs beside the MFMAs of d-tile dt
+      auto rescale = [&](auto ic) __attribute__((always_inline)) {
+        constexpr int dt = decltype(ic)::value;
+        if constexpr (dt < 8) {
+          oacc[dt][0] *= __uint_as_float(al[0]);
+          oacc[dt][1] *= __uint_as_float(al[1]);
+        }
+      };
+      rescale(std::integral_constant<int, 0>{});
+      unroll<0, 8>([&](auto ic) __attribute__((always_inline)) {
+        constexpr int dt = decltype(ic)::value;
+        read_v(std::integral_constant<int, dt + VDEPTH - 1>{});
+        if constexpr (dt >= VDEPTH - 1) {
+          constexpr int ahead = 2 * (7 - dt < VDEPTH - 1 ? 7 - dt : VDEPTH - 1);
+          lgkm_wait<ahead>();
+          landed(vl[dt % VDEPTH]);
+          landed(vh[dt % VDEPTH]);
+        }
+        const u32x4 v = {vl[dt % VDEPTH][0], vl[dt % VDEPTH][1], vh[dt % VDEPTH][0], vh[dt % VDEPTH][1]};
+#pragma unroll
+        for (int hh = 0; hh < 2; ++hh) {
+          const u32x4 p = {pb[hh][0][0], pb[hh][0][1], pb[hh][1][0], pb[hh][1][1]};
+          oacc[dt][hh] = mh_mma<BF16>(v, p, oacc[dt][hh]);
+        }
+        rescale(std::integral_constant<int, dt + 1>{});
+      });
     }
 
-    // ---- end of the piece: row sums over the lane groups and the two token halves
+    // ---- end of the piece: row sums over the lanes of a head
     mh_barrier();  // the exchange area's last readers are done
     {
-      float x = l + __shfl_xor(l, 16, 64);
+      float x = l + mh_ror8(l);
+      x += __shfl_xor(x, 16, 64);
       x += __shfl_xor(x, 32, 64);
-      if (g == 0) ds_put32(x_addr(th, dh), __float_as_uint(x));
+      ds_put32(put_x, __float_as_uint(x));
+      ds_put32(put_x + 32, __float_as_uint(m));
     }
     mh_barrier();
     const bool whole = t0 == 0 && t1 == tiles;
     const int64_t slot = t0 == 0 ? mh_head_slot(a, r, b) : mh_tail_slot(r);
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
-      const float lt = __uint_as_float(ds_get32(x_addr(0, hh))) + __uint_as_float(ds_get32(x_addr(1, hh)));
+      const float lt = __uint_as_float(ds_get32(get_x + 2 * hh * MH_BOX));
       const float inv = lt > 0.f ? 1.0f / lt : 0.f;
       const int head = hb * MH_HEADS + 32 * hg + 16 * hh + jl;
       if (whole) {
@@ -536,8 +549,8 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
         float* const o = a.ws_o + (slot * a.Hq + head) * MH_DV + 128 * w + 4 * g;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) *(f32x4*)(o + 16 * dt) = oacc[dt][hh] * inv;
-        if (w == 0 && g == 0)
-          a.ws_lse[slot * a.Hq + head] = lt > 0.f ? m[hh] + __log2f(lt) : -INFINITY;
+        const float mt = __uint_as_float(ds_get32(get_x + 32 + 2 * hh * MH_BOX));
+        if (w == 0 && g == 0) a.ws_lse[slot * a.Hq + head] = lt > 0.f ? mt + __log2f(lt) : -INFINITY;
       }
     }
   }
