@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string>
+#include <type_traits>
 
 #include "../../include/tlmi355x.h"
 
@@ -116,6 +117,33 @@ TLM_DEV float xhalf_sum(float x) {
                                                   false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+
+// LDS accesses as inline asm, for kernels that keep LDS-DMA loads in flight: compiler-generated ones may be made
+// to wait for every such load. A read's result is used only after a wait for it and landed().
+namespace ldsop {
+TLM_DEV uint32_t lds_u32(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+template <int OFF>
+TLM_DEV void ds_b128(u32x4& r, uint32_t a) {
+  static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(a), "i"(OFF) : "memory");
+}
+template <int OFF>
+TLM_DEV void ds_tr16(u32x2& r, uint32_t a) {
+  static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
+  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(a), "i"(OFF) : "memory");
+}
+TLM_DEV void landed(u32x4& a) { asm volatile("" : "+v"(a)); }
+TLM_DEV void landed(u32x2& a) { asm volatile("" : "+v"(a)); }
+template <int I, int N, typename F>
+TLM_DEV void unroll(F&& f) {  // f(integral_constant) for I .. N - 1
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    unroll<I + 1, N>(f);
+  }
+}
+}  // namespace ldsop
 
 // Non-temporal (streaming) 16-byte global accesses for single-use data.
 TLM_DEV u32x4 ld_nt(const u32x4* p) { return __builtin_nontemporal_load(p); }

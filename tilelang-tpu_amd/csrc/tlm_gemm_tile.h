@@ -75,23 +75,8 @@ struct Cfg {
   static_assert(SMEM <= 160 * 1024, "LDS");
 };
 
-TLM_DEV uint32_t lds_u32(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-// LDS reads as inline asm: compiler-generated ones may be made to wait for every LDS-DMA load in
-// flight. Their results are used only after lgkm_wait0 + landed().
-template <int OFF>
-TLM_DEV void ds_b128(u32x4& r, uint32_t a) {
-  static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(a), "i"(OFF) : "memory");
-}
-template <int OFF>
-TLM_DEV void ds_tr16(u32x2& r, uint32_t a) {
-  static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(a), "i"(OFF) : "memory");
-}
-TLM_DEV void landed(u32x4& a) { asm volatile("" : "+v"(a)); }
-TLM_DEV void landed(u32x2& a) { asm volatile("" : "+v"(a)); }
+using namespace ldsop;
+
 TLM_DEV void lgkm_wait0() {
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_waitcnt(0xc07f);
@@ -109,16 +94,8 @@ TLM_DEV void tile_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int I, int N, typename F>
-TLM_DEV void unroll(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    unroll<I + 1, N>(f);
-  }
-}
-
 // 16-byte chunk c of row r of an [rows][BKB bytes] tile sits at c ^ swz: 16 lanes that read one
-// chunk column of 16 consecutive rows hit 16 different 16-byte banks windows of 256 bytes.
+// chunk column of 16 consecutive rows hit the 16 different 16-byte windows of all banks.
 template <int BKB>
 TLM_DEV int swz_row(int r) {
   return BKB == 128 ? (r >> 1) & 7 : r & 15;

@@ -86,18 +86,7 @@ TLM_DEV f32x4 mh_mma(u32x4 a, u32x4 b, f32x4 c) {
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
-// LDS accesses as inline asm: compiler-generated ones may be made to wait for the LDS-DMA loads of the
-// next tile. Reads are used only after lgkm_wait + landed().
-template <int OFF>
-TLM_DEV void ds_b128(u32x4& r, uint32_t a) {
-  static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(a), "i"(OFF) : "memory");
-}
-template <int OFF>
-TLM_DEV void ds_tr16(u32x2& r, uint32_t a) {
-  static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
-  asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(a), "i"(OFF) : "memory");
-}
+using namespace ldsop;
 template <int OFF>
 TLM_DEV void ds_b64(u32x2& r, uint32_t a) {
   static_assert(OFF >= 0 && OFF < 65536, "ds offset is 16 bits");
@@ -119,8 +108,6 @@ TLM_DEV uint32_t ds_get32(uint32_t a) {  // waits for the value
   asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(r) : "v"(a) : "memory");
   return r;
 }
-TLM_DEV void landed(u32x4& a) { asm volatile("" : "+v"(a)); }
-TLM_DEV void landed(u32x2& a) { asm volatile("" : "+v"(a)); }
 template <int N>
 TLM_DEV void lgkm_wait() {
   static_assert(N >= 0 && N < 16, "lgkmcnt is 4 bits");
@@ -144,17 +131,6 @@ TLM_DEV void mh_barrier() {
 TLM_DEV float mh_ror8(float x) {  // of lane l ^ 8
   return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), 0x128, 0xf, 0xf, false));
 }
-TLM_DEV uint32_t mh_lds(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-template <int I, int N, typename F>
-TLM_DEV void unroll(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    unroll<I + 1, N>(f);
-  }
-}
-
 TLM_DEV int mh_tiles(const MhArgs& a, int b) {
   const int L = max(0, min(a.sl[b], a.max_pages * a.page));
   return (L + MH_BN - 1) / MH_BN;
@@ -263,7 +239,7 @@ __global__ __launch_bounds__(512, 1) void mla_h16_decode(const MhArgs a) {
   if (lo >= hi) return;  // whole workgroup
   int seq_before = start.before;
 
-  const uint32_t s0 = mh_lds(smem);  // 1 KB aligned: the XORs below stay within a row
+  const uint32_t s0 = lds_u32(smem);  // 1 KB aligned: the XORs below stay within a row
   auto f_swz = [](int t) { return ((t & 7) << 1) | ((t >> 3) & 1); };
   // S^T: A operand = K row 16 th + jl, chunk 4 ks + g (rope: chunk g of the rope row): k_a ^ 64 (ks % 4), ks / 4
   // as an immediate
