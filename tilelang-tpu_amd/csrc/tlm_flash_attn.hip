@@ -534,7 +534,7 @@ __global__ __launch_bounds__(512, 1) void fa_fwd_pp(const uint16_t* __restrict__
   if constexpr (SPLIT) {  // workgroup = (internal split, batch, head, query tile)
     // Where no K / V tile is shared and the parts are a multiple of 8, parts innermost would give each XCD one
     // key range of all heads: with the heads innermost instead, 1 x 128 queries, 8,192 keys, 32 heads, 4
-    // splits took 38.4 us a call for 41.2, 2 x 128, 2,048 keys, 8 splits 41.7 for 43.0. With 2 parts it
+    // splits took 36.2 us a call for 40.0, 2 x 128, 2,048 keys, 8 splits 40.0 for 42.7. With 2 parts it
     // was the slower order (4 x 64 queries, 8,192 keys, 1 split: 94.2 us).
     if (NT && sp.nsi % 8 == 0) {
       si = lin / (nslot * B * H);

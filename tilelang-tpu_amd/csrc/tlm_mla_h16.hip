@@ -8,8 +8,8 @@
 // 500 .. 4,000 tokens, 128 heads (bf16): 26.0 us and 8.2 us for the combine, where the split kernel that
 // it replaced took 67.2 and 14.7; 20.7 MB of cache rows would take 3.1 us. Inside a workgroup 1.6 us go to the
 // scan, 5 to the block table and Q, 2.6 to the first tile and 2 to 4 to the partial rows (33 MB of fp32 for
-// 128 ranges, written and read again); the rest is the launch. 16 x 4,000 .. 8,000 tokens: 64.6 us, of which a
-// 32-token tile takes 1.9 with the next ones already there. It has 1,100 cycles of MFMA issue per SIMD
+// 128 ranges, written and read again); the rest is the launch. 16 x 4,000 .. 8,000 tokens: 65 to 67 us, of which
+// a 32-token tile takes 1.9 with the next ones already there. It has 1,100 cycles of MFMA issue per SIMD
 // and 1,450 of LDS reads per CU (K and V^T operands, 140 KB); leaving out the loads or the MFMAs, or
 // taking the rows from L2, changes the kernel's time by less than 5 %: the chain read, multiply, exchange,
 // softmax, barrier is what remains, with two waves per SIMD to overlap it.
