@@ -329,7 +329,7 @@ int tlm_elementwise(const void* const* in, const int* in_dtype, const int* in_bc
  *   a multiple of 64 and Hq a multiple of 64 the decode runs on the fp8 matrix cores with the
  *   sequences' tiles balanced over B*num_split/(Hq/64) ranges (num_split then only sets the
  *   parallelism). A 16-bit cache of up to 4,096 sequences is balanced alike, over about one
- *   workgroup per CU as far as `ws` holds the partial rows; other cases use one workgroup per
+ *   workgroup per CU as far as tlm_mla_workspace_bytes(...) holds the partial rows; other cases use one workgroup per
  *   (sequence, split, 64 heads).
  * dv = 512, dpe = 64, Hq a multiple of 64 and 16-byte aligned Q / KV rows take those
  *   matrix-core kernels; any other dv <= 1024, dpe <= 256, Hq <= 4096 (e.g. the TPU program

@@ -15,7 +15,7 @@ DEV = "cuda"
 DV, DPE = 512, 64
 
 
-def _case(lens, H, page, dt, seed=0, ns=4, fused=True, jump=None, bad_page=False, edit=None):
+def _case(lens, H, page, dt, seed=0, ns=4, fused=True, jump=None, bad_page=False, edit=None, ws_bytes=None):
     g = torch.Generator(device=DEV).manual_seed(seed + sum(lens) + H)
     B = len(lens)
     pages = max(1, -(-max(lens) // page))
@@ -46,7 +46,7 @@ def _case(lens, H, page, dt, seed=0, ns=4, fused=True, jump=None, bad_page=False
     if not fused:
         kv, kpe = kv.contiguous(), kpe.contiguous()
     out = torch.full((B, H, DV), float("nan"), dtype=dt, device=DEV)
-    ws = torch.empty(ops.mla_workspace_bytes(B, H, DV, ns), dtype=torch.uint8, device=DEV)
+    ws = torch.empty(ws_bytes or ops.mla_workspace_bytes(B, H, DV, ns), dtype=torch.uint8, device=DEV)
     ops.mla_decode(q[..., :DV], q[..., DV:], kv, kpe, table, sl, out, ws, page, ns, scale)
     return out, exp
 
@@ -144,3 +144,12 @@ def test_largest_weight_is_exact(at, dt):
     out, exp = _case(lens, 128, 64, dt, edit=edit)
     err = float((out.double() - exp).norm() / exp.norm())
     assert err < 2.0 ** -14, err
+
+
+@pytest.mark.parametrize("lens,H,ns", [([5000], 64, 64), ([7000], 192, 64), ([900, 2000], 64, 16)])
+def test_result_does_not_depend_on_a_larger_workspace(lens, H, ns):
+    """The ranges follow from the call, so a workspace that an earlier, larger call left behind gives the same
+    bits."""
+    need = ops.mla_workspace_bytes(len(lens), H, DV, ns)
+    runs = [_case(lens, H, 64, torch.bfloat16, ns=ns, ws_bytes=b)[0] for b in (need, 2 * need, 128 << 20)]
+    assert torch.equal(runs[1], runs[0]) and torch.equal(runs[2], runs[0])

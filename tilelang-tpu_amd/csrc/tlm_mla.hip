@@ -762,10 +762,11 @@ static int mla_run(const char* fn, const void* q, const void* q_pe, int64_t q_st
   }
   // 8 x 500 .. 4,000 tokens of 128 bf16 heads: 32 us a call, split kernel 77; replayed in a graph, 8 x 4,000
   // with num_split 1 40 against 442, 256 x 500 87 against 186, one sequence of 64 tokens 16 against 33
+  // (the ranges follow from the call's own need, so a larger workspace gives the same bits)
   if (kv_dtype != TLM_F8E4M3) {
     const int rc = tlm_mla_h16_launch(
         q, q_pe, q_stride, q_pe_stride, kv, k_pe, kv_stride, kpe_stride, kv_rows, block_table, seqlens,
-        o, ws, ws_bytes, B, Hq, page,
+        o, ws, std::min(ws_bytes, tlm_mla_workspace_bytes(B, Hq, dv, num_split)), B, Hq, page,
         max_pages, sc, q_dtype == TLM_BF16, o_dtype == TLM_BF16, stream);
     if (rc != TLM_EUNSUPPORTED) return rc;
   }
