@@ -133,13 +133,13 @@ size_t tlm_gemm_swiglu_tmp_bytes(int64_t M, int64_t N, int64_t K);
 int tlm_gemm_swiglu(const void* A, const void* B_gate, const void* B_up, void* H, void* tmp,
                     int64_t M, int64_t N, int64_t K, int dtype, void* stream);
 
-/* What tlm_gemm, tlm_gemm_fp8 (in_dtype F8E4M3 | F8E5M2) or, with dual != 0, tlm_gemm_swiglu runs for a shape
- * on 16-byte aligned operands: the rows and columns of its tile and the number of workgroups that split
- * K. 16 x 128 is the kernel of one decode step, 256 x 256 the one of whole prompt batches (for
- * tlm_gemm_swiglu the three calls), 0 x 0 one thread per output (K or N not whole 16-byte rows, or past
- * the tiles' launch limits). `captured`:
- * the stream is being captured. A call whose stream finds no workspace slot runs as one that may not
- * split. Host only, no HIP call. */
+/* What tlm_gemm, tlm_gemm_fp8 (in_dtype F8E4M3 | F8E5M2) or, with dual != 0, tlm_gemm_swiglu runs
+ * for a shape on 16-byte aligned operands: the rows and columns of its tile and the number of
+ * workgroups that split K. 16 x 128 is the kernel of one decode step, 256 x 256 the one of whole
+ * prompt batches (for tlm_gemm_swiglu the three calls), 0 x 0 one thread per output (K or N not
+ * whole 16-byte rows, or fp8 past the tiles' limits). `captured`: the stream is being captured. A
+ * call whose stream finds no workspace slot runs as one that may not split. Host only, no HIP
+ * call. */
 int tlm_gemm_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int trans_b, int dual, void* stream,
                   int captured, int* rows, int* cols, int* splits);
 
@@ -329,8 +329,8 @@ int tlm_elementwise(const void* const* in, const int* in_dtype, const int* in_bc
  *   a multiple of 64 and Hq a multiple of 64 the decode runs on the fp8 matrix cores with the
  *   sequences' tiles balanced over B*num_split/(Hq/64) ranges (num_split then only sets the
  *   parallelism). A 16-bit cache of up to 4,096 sequences is balanced alike, over about one
- *   workgroup per CU as far as tlm_mla_workspace_bytes(...) holds the partial rows; other cases use one workgroup per
- *   (sequence, split, 64 heads).
+ *   workgroup per CU as far as tlm_mla_workspace_bytes(...) holds the partial rows; other cases
+ *   use one workgroup per (sequence, split, 64 heads).
  * dv = 512, dpe = 64, Hq a multiple of 64 and 16-byte aligned Q / KV rows take those
  *   matrix-core kernels; any other dv <= 1024, dpe <= 256, Hq <= 4096 (e.g. the TPU program
  *   tpu_demo/ppl/deepseek_mla/mla_decode.py at dim 32 + rope 4 over 8 heads) runs a generic
